@@ -1092,7 +1092,12 @@ void mgpu::ewald_charge_adjoint(mgpu_engine *e, const double *v, const double *d
    KcArgs ka{nk, host_det(e->h), -1.0 / (4.0 * e->alpha * e->alpha), 2 * PI_D * e->hinv[8], e->d_rows.p, e->d_krow.p};
    k_kcoeff<<<(nk + 255) / 256, 256, 0, e->stream>>>(ka, kc);
    weighted_sf(e, e->d_chg_site.p, csq);
+   // an id without sites (id 0 in every Moldy system) has zero sums
+   std::vector<char> used(nid, 0);
+   for (int t : e->site_type) used[t] = 1;
+   zero_async(e, csa, sizeof(double2) * nk * (size_t)nid);
    for (int a = 0; a < nid; a++) {
+      if (!used[a]) continue;
       k_site_weight<<<nb, 256, 0, e->stream>>>(ns, 0, a, e->d_site_type.p, e->d_chg_site.p, nullptr, nsp, w);
       weighted_sf(e, w, csa + (size_t)a * nk);
    }

@@ -1,8 +1,8 @@
 // The site-site pair term of the reference's kernel() (src/kernel.c:188-460)
 // for every potential form, templated on the arithmetic type: double and
-// float for the force kernels, Dual<N> for the parameter adjoint (forward-mode
-// derivatives of u and forceij with respect to the pair's parameters and the
-// charge product, carried alongside the value).
+// float for the force kernels, Dual<1> for the constant terms of the parameter
+// adjoint (the derivative of u with respect to one parameter or charge,
+// carried alongside the value).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>

@@ -90,6 +90,40 @@ def test_adjoint_vs_central_differences(case):
     fw.eng.close()
 
 
+@pytest.mark.parametrize("case,subcell", [("argon", 8.5), ("argon", 0.9), ("water", 6.0), ("silica", 3.3), ("large", 0.0)])
+def test_adjoint_occupancies(case, subcell):
+    """Cells of many sites (a lane lists its cell in several rounds), of few
+    (most lanes of a round list none), and a system whose waves take more
+    than one site each; dE/dtheta and the cotangent product against central
+    differences, the directional derivative against their pairing
+    (v . jvp(dtheta) = dtheta . vjp(v)), which is exact in real arithmetic:
+    FP64 sums of at most 1e7 terms, 1e-10."""
+    from moldy_amd import engine as E
+    if case == "large":
+        s = system.argon_fcc(ncell=17, jitter=0.05, cutoff=6.0)
+    else:
+        s = _cases()[case]()
+    s.control.subcell = subcell
+    fw = Forward(s)
+    th = E.get_theta(s)
+    rng = np.random.Generator(np.random.Philox(23))
+    v = rng.standard_normal((3, s.nsites))
+    dth = rng.standard_normal(th.size) * np.abs(th)
+    got = fw.adjoint(th, v=v, dtheta=dth)
+    assert abs((v * got["jvp"]).sum() - dth @ got["vjp"]) < 1e-10 * np.abs(dth * got["vjp"]).sum()
+    alone = fw.adjoint(th)           # no cotangent: the dE half only
+    assert np.array_equal(alone["dE"], got["dE"])
+    h = _steps(th)
+    for t in np.flatnonzero(th)[:4]:
+        tp, tm = th.copy(), th.copy()
+        tp[t] += h[t]
+        tm[t] -= h[t]
+        (ep, fp), (em, fm) = fw(tp), fw(tm)
+        assert abs((ep - em) / (2 * h[t]) - got["dE"][t]) < TOL * np.abs(got["dE"]).max()
+        assert abs((v * (fp - fm)).sum() / (2 * h[t]) - got["vjp"][t]) < TOL * np.abs(got["vjp"]).max()
+    fw.eng.close()
+
+
 def test_force_matching_gradient_through_autograd():
     """Silica-like crystal, Buckingham: loss = |F(theta) - F_target|^2 with
     the target forces of a perturbed parameter set."""
