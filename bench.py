@@ -69,7 +69,8 @@ def time_gpu(eng, steps, warmup):
     prof = {}
     for name in ["binning", "realspace", "ewald_trig", "ewald_sfac", "ewald_kspace",
                  "ewald_force", "ewald_mfma_sk", "ewald_mfma_reduce", "ewald_mfma_force", "ewald_mfma_prep",
-                 "make_sites", "glue"]:
+                 "ewald_grid_spread", "ewald_grid_forward", "ewald_grid_kspace", "ewald_grid_inverse",
+                 "ewald_grid_gather", "make_sites", "glue"]:
         ms, n = eng.profile_get(name)
         if n:
             prof[name] = ms
@@ -401,7 +402,8 @@ def main():
         tmx, profmx = time_gpu(eng, a.steps, a.warmup)
         pemx, _, stmx = eng.eval_forces_device()
         fmx, tqmx, _, sfmx = eng.download()
-        res["mfma_issued_per_launch"] = mfma_issued(eng, s.nsites)
+        if "ewald_mfma_force" in profmx:   # the direct reciprocal sum (small systems, frameworks)
+            res["mfma_issued_per_launch"] = mfma_issued(eng, s.nsites)
         print(f"[bench] mixed {1e3 * tmx:.3f} ms/eval {profmx}", file=sys.stderr, flush=True)
         mixed = dict(t=tmx, prof=profmx,
                      err=dict(site_force=rms_rel(sfmx, sf64), mol_force=rms_rel(fmx, f64),
@@ -429,11 +431,14 @@ def main():
         res["mixed_over_fp64"] = t64 / mixed["t"]
         res["mixed_error_vs_fp64"] = mixed["err"]
     prof = mixed["prof"] if mixed else prof64
-    # roofline of the dominant kernel: the back-projection, the longest kernel
-    # that runs alone (the tables, S(k) and the real-space pass may share the
-    # GPU when the two streams overlap, so their timed durations are not their own)
-    dom = "ewald_mfma_force" if "ewald_mfma_force" in prof else "ewald_force"
-    kind = {"ewald_sfac": ("fp64_mfma", FLOPS_SK_PER_KI * nk * ns),
+    # roofline of the dominant kernel: with the direct reciprocal sum its
+    # back-projection, the longest kernel that runs alone; with the gridded
+    # sum the real-space pass (timed while it shares the GPU with the
+    # reciprocal stages when the two streams overlap)
+    dom = next(k for k in ("ewald_mfma_force", "ewald_force", "realspace") if k in prof)
+    pairs = 0.5 * ns * ns / s.volume() * 4.0 / 3.0 * np.pi * s.control.cutoff ** 3
+    kind = {"realspace": ("fp32_vector" if mixed else "fp64_vector", FLOPS_PER_PAIR * pairs),
+            "ewald_sfac": ("fp64_mfma", FLOPS_SK_PER_KI * nk * ns),
             "ewald_force": ("fp64_vector", FLOPS_FORCE_PER_KI * nk * ns),
             "ewald_mfma_sk": ("fp16_mfma", FLOPS_SK_PER_KI * nk * ns),
             "ewald_mfma_force": ("fp16_mfma", FLOPS_FORCE_PER_KI * nk * ns)}.get(dom)

@@ -1,0 +1,1000 @@
+// Reciprocal-space Ewald sum on a grid (src/ewald.c:280-589): the
+// same finite k set, weights and half-space sums as the direct sum, with the
+// structure factors and the back-projection formed by spreading the charges
+// over a grid with a compact window, transforming the grid, and dividing the
+// window's transform out.
+//
+// The direct sums take N_k N_s complex products (1.3e10 at 132,872 sites);
+// here a site meets w^3 grid points and the transforms cost about 4 n^3 (n/2)
+// multiply-adds in all.  The k set is the direct path's, so nothing is
+// truncated that the reference keeps: the window only approximates
+// exp(i k.r), and its width is set so that the error lies at the rounding of
+// the arithmetic (w = 16 in FP64, w = 8 in FP32; at least 4.6 and 4 grid
+// points per shortest wave in each direction; the sampling theorem asks for 2).
+//
+//   window   phi(z) = exp(beta (sqrt(1 - z^2) - 1)), |z| <= 1, z = 2 d / w for a
+//            grid distance d (the "exponential of semicircle" window of
+//            Barnett, Magland and af Klinteberg, SIAM J. Sci. Comput. 41, C479,
+//            2019).  beta = 2.5 w (FP64) and 2.6 w (FP32): past their 2.3 w,
+//            because the Ewald weight exp(-k^2/4 alpha^2) damps the k next to
+//            the cutoff, whose aliases a larger beta raises, while the
+//            derivative of the window at its edge falls.  It is evaluated as one polynomial per grid offset.
+//   spread   G(x,y,z) = sum_i q_i phi phi phi
+//   forward  T(h,k,l) = sum_xyz G e^{+2 pi i (hx/nx + ky/ny + lz/nz)}, l >= 0, as
+//            dense transforms of one axis at a time on the matrix cores: only the
+//            modes of the k set's box are formed (a quarter of each axis), so
+//            the dense form costs about what a full FFT would
+//   k space  S = T / (phi^ phi^ phi^); energy, stress (ewald.c:539-553); W = coeff S / (phi^ phi^ phi^)
+//   inverse  Phi(x,y,z) = Re sum W e^{-2 pi i (...)}
+//   gather   F_i = -q_i grad sum_g Phi(g) phi phi phi, the gradient of the window's polynomials
+//
+// The transforms (and the window's polynomials) run in FP64 for both: in FP32
+// the transforms' rounding alone made an error of 9.5e-7 in the forces of 729
+// waters (4e-7 for all else), because the sums
+// over the grid cancel; they are a small part of the pass.
+//
+// Every sum has a fixed order (a brick's sites are ranked by index before
+// they are added), so results repeat bit for bit.
+#include "mgpu_internal.h"
+#include "mgpu_ewald_grid.h"
+
+#include <algorithm>
+#include <cmath>
+
+using namespace mgpu;
+
+namespace {
+
+constexpr double PI_D = 3.14159265358979323846;
+constexpr int GB = 8;               // brick edge in grid points
+
+// Window width and polynomial degree of each arithmetic.
+template <class R> struct Win;
+template <> struct Win<double> {
+   static constexpr int W = 16, DEG = 15;
+   static constexpr double BETA = 2.5 * W;
+};
+template <> struct Win<float> {
+   static constexpr int W = 8, DEG = 10;
+   static constexpr double BETA = 2.6 * W;
+};
+// A site's spread weights: three rows of WP = W + 16, the W weights from
+// element 8 and zeros around them, so that a brick reads them at any offset.
+template <class R> constexpr int WP = Win<R>::W + 2 * GB;
+
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+// 16x16x4 matrix product: A row (B column) lane % 16 at k = lane / 16; item v
+// of D is row lane / 16 + 4 v of column lane % 16.
+__device__ __forceinline__ dbl4 mma(double a, double b, dbl4 c) {
+   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+template <class R> struct Vec;
+template <> struct Vec<double> {
+   using T2 = double2;
+};
+template <> struct Vec<float> {
+   using T2 = float2;
+};
+
+// The wave's own LDS writes before its reads.
+__device__ __forceinline__ void wave_lds_sync() {
+   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+   __builtin_amdgcn_wave_barrier();
+   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// ------------------------------------------------------------ binning
+struct GBinArgs {
+   double hinv[9];
+   int n[3], nb[3];      // grid points, bricks
+   int ns, nsp, w, cap;
+   const double *site;
+   int4 *sa;             // per site: anchor (first grid point of the window, wrapped) and brick
+   double *sx;           // per site: polynomial argument per axis, [3][nsp]
+   int *cnt, *bucket;    // per brick: sites seen; [brick][cap] the first cap of them
+};
+
+// Anchor a = ceil(u - w/2) and the polynomials' argument 2 (a - (u - w/2)) - 1
+// of each axis, u the grid coordinate; sites counted into the bricks of
+// their anchors.  The fractional coordinate is formed as a sum of two doubles
+// and the argument with one fma from the anchor: the position within the
+// window then carries no rounding of the size of the box (which would be a
+// phase error growing with |h|, as the trig recurrence of the direct sum has).
+__device__ __forceinline__ void b_g_bin(int bx, int nbx, const GBinArgs &a) {
+#pragma clang fp contract(off)
+   const int i = bx * 256 + threadIdx.x;
+   if (i >= a.ns) return;
+   const double r[3] = {a.site[i], a.site[a.nsp + i], a.site[2 * (size_t)a.nsp + i]};
+   int an[3];
+#pragma unroll
+   for (int d = 0; d < 3; d++) {
+      double hi = 0, lo = 0;
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+         const double p = a.hinv[3 * d + c] * r[c];
+         lo += __builtin_fma(a.hinv[3 * d + c], r[c], -p);
+         const double t = hi + p, z = t - hi;
+         lo += (hi - (t - z)) + (p - z);
+         hi = t;
+      }
+      hi -= rint(hi);
+      if (!(fabs(hi) <= 0.5)) hi = lo = 0.0;   // not a number
+      const double n = a.n[d], hw = 0.5 * a.w, c = ceil(__builtin_fma(n, hi, -hw));
+      an[d] = (int)c;
+      if (an[d] < 0) an[d] += a.n[d];
+      a.sx[(size_t)d * a.nsp + i] = 2.0 * (__builtin_fma(-n, hi, c + hw) - n * lo) - 1.0;
+   }
+   const int b = ((an[0] / GB) * a.nb[1] + an[1] / GB) * a.nb[2] + an[2] / GB;
+   a.sa[i] = make_int4(an[0], an[1], an[2], b);
+   const int slot = atomicAdd(&a.cnt[b], 1);
+   if (slot < a.cap) a.bucket[(size_t)b * a.cap + slot] = i;
+}
+__global__ __launch_bounds__(256) void k_g_bin(GBinArgs a) { b_g_bin(blockIdx.x, gridDim.x, a); }
+
+// Exclusive prefix sum of the brick counts, one block.
+__device__ __forceinline__ void b_g_scan(int bx, int nbx, int nb, const int *__restrict__ cnt,
+                                         int *__restrict__ start) {
+   __shared__ int ws[4];
+   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+   const int per = (nb + 255) / 256, b0 = min(t * per, nb), b1 = min(b0 + per, nb);
+   int s = 0;
+   for (int b = b0; b < b1; b++) s += cnt[b];
+   const int inc = wave_incl_scan(s, lane);
+   if (lane == 63) ws[wv] = inc;
+   __syncthreads();
+   int off = inc - s;
+   for (int q = 0; q < wv; q++) off += ws[q];
+   for (int b = b0; b < b1; b++) {
+      start[b] = off;
+      off += cnt[b];
+   }
+   if (t == 255) start[nb] = off;
+}
+__global__ __launch_bounds__(256) void k_g_scan(int nb, const int *__restrict__ cnt, int *__restrict__ start) {
+   b_g_scan(blockIdx.x, gridDim.x, nb, cnt, start);
+}
+
+// ------------------------------------------------------------ weights
+struct GWtArgs {
+   int nb, ns, nsp, cap;
+   const int4 *sa;
+   const double *sx, *chg;
+   const int *bucket, *start;
+   int *cnt;             // cleared for the next pass
+   const double *poly;   // [DEG + 1][W]
+   void *wt;             // R [ns][3][WP], pads already zero
+   int4 *anc;            // brick order: anchor and site index
+   double4 *fr;          // [ns]: arguments and charge
+};
+
+// One wave per brick: its sites in index order, each with its anchor,
+// arguments and spread weights (the charge in the x row).  A brick with more
+// than cap sites collects them by a walk over all sites.
+template <class R>
+__device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
+   constexpr int W = Win<R>::W, DEG = Win<R>::DEG, NL = 3 * W;
+   extern __shared__ double gw_lds[];
+   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+   const int b = bx * 4 + wave;
+   if (b >= a.nb) return;   // wave-uniform; no block barrier in this kernel
+   double *xs = gw_lds + wave * 4 * a.cap;                  // the ranked sites' arguments and charges
+   int *list = (int *)(gw_lds + 16 * a.cap) + wave * a.cap;
+   const int m = a.cnt[b], s0 = a.start[b];
+   // lanes d * W + p: the polynomial of offset p on axis d
+   double c[DEG + 1];
+   const int wd = lane / W, wp = lane % W;
+#pragma unroll
+   for (int k = 0; k <= DEG; k++) c[k] = lane < NL ? a.poly[k * W + wp] : 0.0;
+   auto place = [&](int i, int pos) {
+      const int4 s = a.sa[i];
+      a.anc[pos] = make_int4(s.x, s.y, s.z, i);
+      const double4 f = make_double4(a.sx[i], a.sx[(size_t)a.nsp + i], a.sx[2 * (size_t)a.nsp + i], a.chg[i]);
+      a.fr[pos] = f;
+      return f;
+   };
+   auto weights = [&](double x, double q, int pos) {
+      double v = c[DEG];
+#pragma unroll
+      for (int k = DEG - 1; k >= 0; k--) v = v * x + c[k];
+      if (wd == 0) v *= q;
+      if (lane < NL) ((R *)a.wt)[((size_t)pos * 3 + wd) * WP<R> + GB + wp] = (R)v;
+   };
+   if (m <= a.cap) {
+      for (int t = lane; t < m; t += 64) list[t] = a.bucket[(size_t)b * a.cap + t];
+      wave_lds_sync();
+      for (int t = lane; t < m; t += 64) {
+         const int i = list[t];
+         int r = 0;
+         for (int q = 0; q < m; q++) r += list[q] < i;
+         const double4 f = place(i, s0 + r);
+         xs[4 * r] = f.x;
+         xs[4 * r + 1] = f.y;
+         xs[4 * r + 2] = f.z;
+         xs[4 * r + 3] = f.w;
+      }
+      wave_lds_sync();
+      for (int t = 0; t < m; t++) weights(xs[4 * t + min(wd, 2)], xs[4 * t + 3], s0 + t);
+   } else {
+      int r = 0;
+      for (int i0 = 0; i0 < a.ns; i0 += 64) {
+         const int i = i0 + lane;
+         const bool in = i < a.ns && a.sa[i].w == b;
+         unsigned long long mk = __ballot(in);
+         if (in) place(i, s0 + r + __popcll(mk & ((1ull << lane) - 1)));
+         for (; mk; mk &= mk - 1, r++) {
+            const int j = i0 + __builtin_ctzll(mk);
+            weights(a.sx[(size_t)min(wd, 2) * a.nsp + j], a.chg[j], s0 + r);
+         }
+      }
+   }
+   if (lane == 0) a.cnt[b] = 0;
+}
+template <class R> __global__ __launch_bounds__(256) void k_g_weights(GWtArgs a) {
+   b_g_weights<R>(blockIdx.x, gridDim.x, a);
+}
+
+// ------------------------------------------------------------ spread
+struct GSpArgs {
+   int n[3], nb[3];
+};
+
+// One block per brick of 8^3 grid points; a lane holds the 8 points of one
+// (y, z) in registers.  The sites whose windows reach the brick have their
+// anchors in the W/8 + 1 (W = 16) or 2 (W = 8) bricks per axis up to it; the
+// four waves take every fourth of them.  A site's x weights are wave-uniform
+// (scalar loads), its y and z weights one load each, so a site costs a wave
+// about ten vector instructions for 512 points.
+template <class R>
+__device__ __forceinline__ void b_g_spread(int bx, int nbx, const GSpArgs &a, const R *__restrict__ wt,
+                                           const int4 *__restrict__ anc, const int *__restrict__ start,
+                                           R *__restrict__ G) {
+   constexpr int W = Win<R>::W, P = WP<R>, NK = W > GB + 1 ? 3 : 2;
+   __shared__ R red[4][512];
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int ly = lane >> 3, lz = lane & 7;
+   const int nby = a.nb[1], nbz = a.nb[2];
+   const int Bx = bx / (nby * nbz), By = bx / nbz - nby * Bx, Bz = bx - nbz * (By + nby * Bx);
+   const int zlo = Bz - (NK - 1);
+   R acc[GB];
+#pragma unroll
+   for (int r = 0; r < GB; r++) acc[r] = 0;
+   auto off = [](int base, int an, int n) {
+      int d = base - an;
+      if (d < -(GB - 1)) d += n;
+      return d + GB;
+   };
+   for (int ix = 0; ix < NK; ix++) {
+      const int cx = Bx - ix < 0 ? Bx - ix + a.nb[0] : Bx - ix;
+      for (int iy = 0; iy < NK; iy++) {
+         const int cy = By - iy < 0 ? By - iy + nby : By - iy;
+         const int cb = (cx * nby + cy) * nbz;
+         // the z run of bricks, in two pieces where it wraps
+         for (int pc = 0; pc < (zlo < 0 ? 2 : 1); pc++) {
+            const int z0 = pc == 0 ? max(zlo, 0) : zlo + nbz, z1 = pc == 0 ? Bz + 1 : nbz;
+            const int s = start[cb + z0], e = start[cb + z1];
+            int j = s + ((wave - s) & 3);
+            auto add = [&](const int4 A, int jj) {
+               const R *wr = wt + (size_t)jj * (3 * P);
+               const R *wx = wr + off(GB * Bx, A.x, a.n[0]);
+               const R wy = wr[P + off(GB * By, A.y, a.n[1]) + ly], wz = wr[2 * P + off(GB * Bz, A.z, a.n[2]) + lz];
+               const R t = wy * wz;
+#pragma unroll
+               for (int r = 0; r < GB; r++) acc[r] += wx[r] * t;
+            };
+            for (; j + 12 < e; j += 16) {
+               int4 A[4];
+#pragma unroll
+               for (int u = 0; u < 4; u++) A[u] = anc[j + 4 * u];
+#pragma unroll
+               for (int u = 0; u < 4; u++) add(A[u], j + 4 * u);
+            }
+            for (; j < e; j += 4) add(anc[j], j);
+         }
+      }
+   }
+#pragma unroll
+   for (int r = 0; r < GB; r++) red[wave][r * 64 + lane] = acc[r];
+   __syncthreads();
+   for (int t = threadIdx.x; t < 512; t += 256) {
+      const int x = GB * Bx + (t >> 6), y = GB * By + ((t >> 3) & 7), z = GB * Bz + (t & 7);
+      G[((size_t)x * a.n[1] + y) * a.n[2] + z] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+   }
+}
+template <class R>
+__global__ __launch_bounds__(256) void k_g_spread(GSpArgs a, const R *__restrict__ wt, const int4 *__restrict__ anc,
+                                                  const int *__restrict__ start, R *__restrict__ G) {
+   b_g_spread<R>(blockIdx.x, gridDim.x, a, wt, anc, start, G);
+}
+
+// ------------------------------------------------------------ transforms
+struct GzArgs {
+   int nlines, K, lda;        // rows of the input, its K and row stride (elements)
+   int ncols, ldt, ldo;       // columns out, table row stride, output row stride
+   int nmt, ngrp;             // row tiles, column groups
+};
+
+// out[line][col] = sum_k in[line][k] tab[k][col]: the z transforms, both
+// ways.  A wave takes 16 lines by NT column tiles; lane (row, g) reads
+// elements 2 g, 2 g + 1 of each 8 (the table's rows taken alike).  The table
+// has zero rows up to a multiple of 8 and zero columns up to whole groups.
+template <class RI, class RO, int NT>
+__device__ __forceinline__ void b_gz(int bx, int nbx, const GzArgs &a, const RI *__restrict__ in,
+                                     const double *__restrict__ tab, RO *__restrict__ out) {
+   using T2 = typename Vec<RI>::T2;
+   const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+   const int t = bx * 4 + (threadIdx.x >> 6);
+   if (t >= a.nmt * a.ngrp) return;
+   const int mt = t / a.ngrp, c0 = (t - mt * a.ngrp) * NT * 16 + m;
+   const RI *ap = in + (size_t)min(mt * 16 + m, a.nlines - 1) * a.lda;
+   dbl4 acc[NT];
+#pragma unroll
+   for (int c = 0; c < NT; c++) acc[c] = dbl4{0, 0, 0, 0};
+   for (int k0 = 0; k0 < a.K; k0 += 8) {
+      const int k = k0 + 2 * g;
+      const T2 av = *(const T2 *)(ap + min(k, a.K - 2));   // K is even
+      const double *tp = tab + (size_t)k * a.ldt + c0;
+#pragma unroll
+      for (int c = 0; c < NT; c++) {
+         acc[c] = mma(av.x, tp[16 * c], acc[c]);
+         acc[c] = mma(av.y, tp[a.ldt + 16 * c], acc[c]);
+      }
+   }
+#pragma unroll
+   for (int v = 0; v < 4; v++) {
+      const int line = mt * 16 + g + 4 * v;
+      if (line >= a.nlines) continue;
+#pragma unroll
+      for (int c = 0; c < NT; c++)
+         if (c0 + 16 * c < a.ncols) out[(size_t)line * a.ldo + c0 + 16 * c] = (RO)acc[c][v];
+   }
+}
+template <class RI, class RO, int NT>
+__global__ __launch_bounds__(256) void k_gz(GzArgs a, const RI *__restrict__ in, const double *__restrict__ tab,
+                                            RO *__restrict__ out) {
+   b_gz<RI, RO, NT>(blockIdx.x, gridDim.x, a, in, tab, out);
+}
+
+struct GcArgs {
+   int nbatch, nmt, nct;             // batches, row tiles, column tiles
+   int K, M, N, ldt;                 // contraction length, rows with an image, columns, table row stride
+   int off, qoff, mq;                // output index of row m: off + m, and qoff - m for 0 < m < mq
+   size_t inb, ink, inc, outb, outm, outc;
+};
+
+// out[b][index(m)][n] = sum_k E[m][k] in[b][k][n] over complex planes (real at
+// 0, imaginary at inc / outc), with the mirrored row conj(E[m]) from the same
+// four real products: the x and y transforms, both ways.  A wave takes one
+// 16 x 16 tile.
+__device__ __forceinline__ void b_gc(int bx, int nbx, const GcArgs &a, const double *__restrict__ in,
+                                     const double *__restrict__ er, const double *__restrict__ ei, double *__restrict__ out) {
+   const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+   const int t = bx * 4 + (threadIdx.x >> 6);
+   if (t >= a.nbatch * a.nmt * a.nct) return;
+   const int b = t / (a.nmt * a.nct), r = t - b * (a.nmt * a.nct), ct = r / a.nmt, mt = r - ct * a.nmt;
+   const int n = ct * 16 + m;
+   const double *ip = in + b * a.inb + min(n, a.N - 1);
+   const double *rp = er + mt * 16 + m, *xp = ei + mt * 16 + m;
+   dbl4 rr{0, 0, 0, 0}, ii{0, 0, 0, 0}, ri{0, 0, 0, 0}, ir{0, 0, 0, 0};
+   for (int k0 = 0; k0 < a.K; k0 += 4) {
+      const int k = k0 + g, kc = min(k, a.K - 1);   // the table's rows past K are zero
+      const double br = ip[kc * a.ink], bi = ip[kc * a.ink + a.inc];
+      const double ar = rp[(size_t)k * a.ldt], ai = xp[(size_t)k * a.ldt];
+      rr = mma(ar, br, rr);
+      ii = mma(ai, bi, ii);
+      ri = mma(ar, bi, ri);
+      ir = mma(ai, br, ir);
+   }
+   if (n >= a.N) return;
+#pragma unroll
+   for (int v = 0; v < 4; v++) {
+      const int mm = mt * 16 + g + 4 * v;
+      if (mm >= a.M) continue;
+      double *o = out + b * a.outb + (size_t)(a.off + mm) * a.outm + n;
+      o[0] = rr[v] - ii[v];
+      o[a.outc] = ri[v] + ir[v];
+      if (mm > 0 && mm < a.mq) {
+         o = out + b * a.outb + (size_t)(a.qoff - mm) * a.outm + n;
+         o[0] = rr[v] + ii[v];
+         o[a.outc] = ri[v] - ir[v];
+      }
+   }
+}
+__global__ __launch_bounds__(256) void k_gc(GcArgs a, const double *__restrict__ in, const double *__restrict__ er,
+                                            const double *__restrict__ ei, double *__restrict__ out) {
+   b_gc(blockIdx.x, gridDim.x, a, in, er, ei, out);
+}
+
+// ------------------------------------------------------------ k space
+struct GkArgs {
+   int hmax, kmax, lmax;
+   double vol, r4a, c2;
+   const KRow *rows;
+   const int *rowmap;              // [hmax + 1][2 kmax + 1]: row of (h, k) or -1
+   const double *dx, *dy, *dz;     // 1 / phi^ per |h|, |k|, |l|
+   double *bpart;                  // [blocks][8]
+};
+
+// Per mode (h, k, l >= 0): energy and stress of the k vector it stands for
+// (itself, or its inverse where the half-space set holds that), and the
+// weight of the inverse transform in its place; modes outside the set become
+// zero.
+__device__ __forceinline__ void b_gk(int bx, int nbx, const GkArgs &a, double *__restrict__ T) {
+   __shared__ double ws[4][8];
+   const int L = a.lmax + 1, NKk = 2 * a.kmax + 1, P = NKk * L;
+   const int e = bx * 256 + threadIdx.x;
+   double v[7] = {0, 0, 0, 0, 0, 0, 0};
+   if (e < (2 * a.hmax + 1) * P) {
+      const int hs = e / P, q = e - hs * P, ks = q / L, l = q - ks * L, h = hs - a.hmax;
+      int r = h >= 0 ? a.rowmap[h * NKk + ks] : -1, ll = l;
+      if (r >= 0 && !(l >= a.rows[r].l0 && l < a.rows[r].l0 + a.rows[r].nl)) r = -1;
+      if (r < 0 && l > 0 && h <= 0) {
+         r = a.rowmap[-h * NKk + 2 * a.kmax - ks];
+         ll = -l;
+         if (r >= 0 && !(ll >= a.rows[r].l0 && ll < a.rows[r].l0 + a.rows[r].nl)) r = -1;
+      }
+      double *p = T + (size_t)hs * 2 * P + q;
+      double wr = 0, wi = 0;
+      if (r >= 0) {
+         const KRow Q = a.rows[r];
+         const double dec = a.dx[h < 0 ? -h : h] * a.dy[ks < a.kmax ? a.kmax - ks : ks - a.kmax] * a.dz[l];
+         const double c = dec * p[0], s = dec * p[P];
+         const double kx = Q.kx, ky = Q.ky, kz = Q.kzt + ll * a.c2;
+         const double ksq = kx * kx + ky * ky + kz * kz;
+         const double coeff = 2.0 / ((0.25 / PI_D) * a.vol) * exp(ksq * a.r4a) / ksq;
+         const double coeff2 = 2.0 * (1.0 - ksq * a.r4a) / ksq;
+         const double pe_k = 0.5 * coeff * (c * c + s * s);
+         v[0] = pe_k;
+         v[1] = pe_k - pe_k * coeff2 * kx * kx;
+         v[2] = -pe_k * coeff2 * kx * ky;
+         v[3] = -pe_k * coeff2 * kx * kz;
+         v[4] = pe_k - pe_k * coeff2 * ky * ky;
+         v[5] = -pe_k * coeff2 * ky * kz;
+         v[6] = pe_k - pe_k * coeff2 * kz * kz;
+         wr = coeff * dec * c;
+         wi = coeff * dec * s;
+      }
+      p[0] = wr;
+      p[P] = wi;
+   }
+   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+   for (int q = 0; q < 7; q++) {
+      const double t = wave_sum(v[q]);
+      if (lane == 0) ws[wv][q] = t;
+   }
+   __syncthreads();
+   if (threadIdx.x < 8)
+      a.bpart[8 * (size_t)bx + threadIdx.x] =
+          threadIdx.x == 7 ? 0.0
+                           : ws[0][threadIdx.x] + ws[1][threadIdx.x] + ws[2][threadIdx.x] + ws[3][threadIdx.x];
+}
+__global__ __launch_bounds__(256) void k_gk(GkArgs a, double *__restrict__ T) {
+   b_gk(blockIdx.x, gridDim.x, a, T);
+}
+
+// ------------------------------------------------------------ gather
+struct GGaArgs {
+   int n[3];
+   int ns, per;          // sites; blocks of each XCD
+   double m[9];          // force = q sum_d G_d m[d]: 2 n_d hinv[d]
+   int nsp, add;         // add: accumulate into out
+};
+constexpr int GA_SPW = 4;   // sites a wave takes in turn
+
+// One wave per site (4 in turn, brick order, so that neighbours share the
+// grid lines they read; consecutive blocks on one XCD).  A lane holds a
+// (y, z) of the window and walks x; the weights and their derivatives come
+// from one polynomial a lane through LDS.
+template <class R>
+__device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, const R *__restrict__ G,
+                                           const double *__restrict__ poly, const int4 *__restrict__ anc,
+                                           const double4 *__restrict__ fr, double *__restrict__ out) {
+   constexpr int W = Win<R>::W, DEG = Win<R>::DEG, NL = 3 * W, LY = 64 / W, NJ = W / LY;
+   using T2 = typename Vec<R>::T2;
+   __shared__ T2 sv[4][NL];
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int wd = lane / W, wp = lane % W;
+   const int blk = (bx & 7) * a.per + (bx >> 3);
+   double c[DEG + 1];
+#pragma unroll
+   for (int k = 0; k <= DEG; k++) c[k] = lane < NL ? poly[k * W + wp] : 0.0;
+   for (int q = 0; q < GA_SPW; q++) {
+      const int pos = (blk * 4 + wave) * GA_SPW + q;
+      if (pos >= a.ns) return;   // wave-uniform; no block barrier in this kernel
+      const int4 A = anc[pos];
+      const double4 f = fr[pos];
+      const double x = wd == 0 ? f.x : wd == 1 ? f.y : f.z;
+      double v = c[DEG], dv = 0;
+#pragma unroll
+      for (int k = DEG - 1; k >= 0; k--) {
+         dv = dv * x + v;
+         v = v * x + c[k];
+      }
+      wave_lds_sync();
+      if (lane < NL) {
+         T2 t;
+         t.x = (R)v;
+         t.y = (R)dv;
+         sv[wave][lane] = t;
+      }
+      wave_lds_sync();
+      int zz = A.z + wp;
+      if (zz >= a.n[2]) zz -= a.n[2];
+      int o[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+         int yy = A.y + j * LY + wd;
+         if (yy >= a.n[1]) yy -= a.n[1];
+         o[j] = yy * a.n[2] + zz;
+      }
+      R a0[NJ], a1[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; j++) a0[j] = a1[j] = 0;
+#pragma unroll
+      for (int i = 0; i < W; i++) {
+         int xx = A.x + i;
+         if (xx >= a.n[0]) xx -= a.n[0];
+         const R *gp = G + (size_t)xx * a.n[1] * a.n[2];
+         const T2 wx = sv[wave][i];
+#pragma unroll
+         for (int j = 0; j < NJ; j++) {
+            const R gv = gp[o[j]];
+            a0[j] += wx.x * gv;
+            a1[j] += wx.y * gv;
+         }
+      }
+      double px = 0, py = 0, p0 = 0;
+#pragma unroll
+      for (int j = 0; j < NJ; j++) {
+         const T2 wy = sv[wave][W + j * LY + wd];
+         px += (double)wy.x * (double)a1[j];
+         py += (double)wy.y * (double)a0[j];
+         p0 += (double)wy.x * (double)a0[j];
+      }
+      const T2 wz = sv[wave][2 * W + wp];
+      const double gx = wave_sum(px * (double)wz.x), gy = wave_sum(py * (double)wz.x),
+                   gz = wave_sum(p0 * (double)wz.y);
+      if (lane < 3) {
+         const double fc = f.w * (gx * a.m[lane] + gy * a.m[3 + lane] + gz * a.m[6 + lane]);
+         double *op = out + (size_t)lane * a.nsp + A.w;
+         *op = a.add ? *op + fc : fc;
+      }
+   }
+}
+template <class R>
+__global__ __launch_bounds__(256) void k_g_gather(GGaArgs a, const R *__restrict__ G,
+                                                  const double *__restrict__ poly, const int4 *__restrict__ anc,
+                                                  const double4 *__restrict__ fr, double *__restrict__ out) {
+   b_g_gather<R>(blockIdx.x, gridDim.x, a, G, poly, anc, fr, out);
+}
+
+// force += the gathered forces, once the real-space pass has added its own.
+__device__ __forceinline__ void b_g_add(int bx, int nbx, int ns, int nsp, const double *__restrict__ f,
+                                        double *__restrict__ force) {
+   const int i = bx * 256 + threadIdx.x;
+   if (i >= ns) return;
+#pragma unroll
+   for (int c = 0; c < 3; c++) force[(size_t)c * nsp + i] += f[(size_t)c * nsp + i];
+}
+__global__ __launch_bounds__(256) void k_g_add(int ns, int nsp, const double *__restrict__ f,
+                                               double *__restrict__ force) {
+   b_g_add(blockIdx.x, gridDim.x, ns, nsp, f, force);
+}
+
+// ------------------------------------------------------------ the plan
+typedef long double ld;
+const ld PI_L = 3.14159265358979323846264338327950288L;
+
+int up(int v, int m) { return (v + m - 1) / m * m; }
+
+ld window(ld z, ld beta) {
+   const ld y = 1.0L - z * z;
+   return y > 0 ? expl(beta * (sqrtl(y) - 1.0L)) : (y == 0 ? expl(-beta) : 0.0L);
+}
+
+// The window's polynomials: for offset p and argument x in [-1, 1], z = (p +
+// (x + 1)/2) / (w/2) - 1; Chebyshev interpolation of degree deg, as monomials.
+template <class R> std::vector<double> window_polys() {
+   constexpr int W = Win<R>::W, N = Win<R>::DEG + 1;
+   const ld beta = Win<R>::BETA;
+   ld T[N][N] = {}, cs[4 * N];
+   T[0][0] = 1;
+   T[1][1] = 1;
+   for (int k = 2; k < N; k++)
+      for (int j = 0; j < N; j++) T[k][j] = (j > 0 ? 2 * T[k - 1][j - 1] : 0) - T[k - 2][j];
+   for (int q = 0; q < 4 * N; q++) cs[q] = cosl(q * PI_L / (2 * N));
+   std::vector<double> out((size_t)N * W);
+   for (int p = 0; p < W; p++) {
+      ld f[N], mono[N] = {};
+      for (int j = 0; j < N; j++) f[j] = window((p + (cs[2 * j + 1] + 1) / 2) / (W / 2.0L) - 1, beta);
+      for (int k = 0; k < N; k++) {
+         ld c = 0;
+         for (int j = 0; j < N; j++) c += f[j] * cs[k * (2 * j + 1) % (4 * N)];
+         c *= (k ? 2.0L : 1.0L) / N;
+         for (int j = 0; j < N; j++) mono[j] += c * T[k][j];
+      }
+      for (int k = 0; k < N; k++) out[(size_t)k * W + p] = (double)mono[k];
+   }
+   return out;
+}
+
+// 1 / phi^(m), phi^(m) = int phi(2 d / w) cos(2 pi m d / n) dd, m = 0 .. mmax, by
+// the tanh-sinh rule (the window has square-root ends); cos(m t) by the
+// three-term recurrence.
+void window_inverse(int w, ld beta, int n, int mmax, std::vector<double> &out) {
+   const ld h = 0.0275L;
+   std::vector<ld> sum(mmax + 1, 0);
+   for (int j = 0; j <= 120; j++) {
+      const ld t = j * h, u = PI_L / 2 * sinhl(t), ch = coshl(u);
+      const ld wt = (j ? 2 : 1) * h * PI_L / 2 * coshl(t) / (ch * ch) * expl(beta * (1 / ch - 1));
+      const ld c1 = cosl(PI_L * w / n * tanhl(u));
+      ld c0 = 1, c = c1;
+      sum[0] += wt;
+      for (int m = 1; m <= mmax; m++) {
+         sum[m] += wt * c;
+         const ld cn = 2 * c1 * c - c0;
+         c0 = c;
+         c = cn;
+      }
+   }
+   for (int m = 0; m <= mmax; m++) out.push_back((double)(1 / (sum[m] * w / 2)));
+}
+
+// Table [rows][ldt] of sign times cos or sin (2 pi r c / n) for r < nr, c < nc (r
+// taken from r0), zero elsewhere.  co holds cos(2 pi j / n); n is a multiple of 4.
+void trig_table(std::vector<double> &out, const std::vector<double> &co, int n, int rows, int ldt, int r0, int nr,
+                int nc, bool sine, double sign) {
+   const size_t o = out.size();
+   out.resize(o + (size_t)rows * ldt, 0.0);
+   for (int r = 0; r < nr; r++) {
+      const int step = ((r0 + r) % n + n) % n;
+      int q = sine ? 3 * n / 4 : 0;   // sin x = cos(x - pi/2)
+      double *row = &out[o + (size_t)r * ldt];
+      for (int c = 0; c < nc; c++) {
+         row[c] = sign * co[q];
+         q += step;
+         if (q >= n) q -= n;
+      }
+   }
+}
+
+std::vector<double> roots(int n) {
+   std::vector<double> co(n);
+   for (int j = 0; j < n; j++) co[j] = 4 * j == n || 4 * j == 3 * n ? 0.0 : (double)cosl(2 * PI_L * j / n);
+   return co;
+}
+
+}  // namespace
+
+GridGeom mgpu::grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const double h[9], const double hinv[9],
+                         double vol, double alpha, double kc, bool fp64) {
+   GridGeom g;
+   g.ns = ns; g.nsp = nsp; g.fp64 = fp64;
+   g.m[0] = hmax; g.m[1] = kmax; g.m[2] = lmax;
+   for (int d = 0; d < 3; d++) {
+      // grid points per shortest wave along this cell vector (kc |h_d| / 2 pi
+      // waves): the aliases of the modes next to the cutoff are down by
+      // phi^(n - m) / phi^(m) = 3e-14 at 4.6 (FP64), 2e-5 at 4 (FP32), before
+      // the weight's own 1e-6
+      const double wv = kc / (2 * PI_D) * sqrt(h[d] * h[d] + h[3 + d] * h[3 + d] + h[6 + d] * h[6 + d]);
+      g.n[d] = (int)std::min(1e6, std::max(3.0 * GB, ceil((fp64 ? 4.6 : 4.0) * wv / GB) * GB));
+      g.nb[d] = g.n[d] / GB;
+   }
+   for (int i = 0; i < 9; i++) g.hinv[i] = hinv[i];
+   g.vol = vol; g.alpha = alpha;
+   g.w = fp64 ? Win<double>::W : Win<float>::W;
+   const long nbr = (long)g.nb[0] * g.nb[1] * g.nb[2];
+   g.cap = up((int)std::min(448L, std::max(64L, 4 * (ns / nbr + 1))), 64);
+   return g;
+}
+
+bool mgpu::grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const std::vector<KRow> &rows) {
+   // frameworks need two structure factors a k; the window's width counts on
+   // the Gaussian damping of the last k; one row per (h, k) is the reference's set
+   if (nsxf != g.ns || g.ns < 1 || rows.empty()) return false;
+   if (!(exp(-kc * kc / (4 * g.alpha * g.alpha)) <= 1e-5)) return false;
+   for (size_t r = 1; r < rows.size(); r++)
+      if (rows[r].h == rows[r - 1].h && rows[r].k == rows[r - 1].k) return false;
+   for (int d = 0; d < 3; d++)
+      if (g.n[d] > 512 || g.n[d] < 4 * g.m[d]) return false;
+   return grid_pays(g, nk);
+}
+
+// Where the grid beats the direct sum: its thirteen launches and its small
+// transforms cost a floor that N_k N_s products must outweigh.  MD step, direct
+// against grid: FP64 water, 8,800 sites (5.4e7 products) 218 and 256 us, 16,384
+// (1.9e8) 346 and 298, 120,000 (1.0e10) 6,404 and 1,113; mixed, 16,384 sites 185
+// and 220 us, 24,000 silica sites (8.2e8) 270 and 266, 120,000 1,053 and 627.
+bool mgpu::grid_pays(const GridGeom &g, int nk) {
+   const double direct = (double)nk * g.ns;
+   return direct > (g.fp64 ? 1.2e8 : 6e8);
+}
+
+GridSizes mgpu::grid_sizes(const GridGeom &g) {
+   GridSizes z;
+   const size_t rs = g.fp64 ? 8 : 4, ns = g.ns;
+   const int wp = g.w + 2 * GB;
+   const size_t L = g.m[2] + 1, P = (2 * g.m[1] + 1) * L;
+   const size_t nb = (size_t)g.nb[0] * g.nb[1] * g.nb[2];
+   size_t off = 0;
+   auto take = [&](size_t bytes) {
+      const size_t o = off;
+      off += (bytes + 255) & ~(size_t)255;
+      return o;
+   };
+   z.sa = take(16 * ns);
+   z.sx = take(8 * 3 * (size_t)g.nsp);
+   z.cnt = take(4 * nb);
+   z.start = take(4 * (nb + 1));
+   z.bucket = take(4 * nb * g.cap);
+   z.anc = take(16 * ns);
+   z.fr = take(32 * ns);
+   z.wt = take(3 * (size_t)wp * rs * ns);
+   z.wt_bytes = 3 * (size_t)wp * rs * ns;
+   z.G = take(rs * g.n[0] * g.n[1] * g.n[2]);
+   z.T1 = take(8 * g.n[0] * g.n[1] * 2 * L);
+   z.T2 = take(8 * g.n[0] * 2 * P);
+   z.T3 = take(8 * (2 * g.m[0] + 1) * 2 * P);
+   z.nred = (int)(((2 * g.m[0] + 1) * P + 255) / 256);
+   z.bpart = take(8 * 8 * (size_t)z.nred);
+   z.fout = take(8 * 3 * (size_t)g.nsp);
+   z.bytes = off;
+   return z;
+}
+
+namespace {
+// Column tiles of a z transform: groups of NT <= 5 tiles.
+void z_split(int ncols, int &nt, int &ngrp) {
+   const int tiles = (ncols + 15) / 16;
+   ngrp = (tiles + 4) / 5;
+   nt = (tiles + ngrp - 1) / ngrp;
+}
+
+template <class R> void build_tables(const GridGeom &g, GridTables &t) {
+   const int W = Win<R>::W, L = g.m[2] + 1;
+   std::vector<double> tab, dec;
+   for (int d = 0; d < 3; d++) {
+      int same = 0;   // an earlier axis of the same grid and box
+      while (same < d && (g.n[same] != g.n[d] || g.m[same] != g.m[d])) same++;
+      t.dec_off[d] = same < d ? t.dec_off[same] : dec.size();
+      if (same == d) window_inverse(W, Win<R>::BETA, g.n[d], g.m[d], dec);
+   }
+   int nt, ng;
+   {   // z: forward [z][c L + l], inverse [c L + l][z]
+      const int n = g.n[2];
+      const std::vector<double> co = roots(n);
+      z_split(2 * L, nt, ng);
+      t.zf_ld = nt * ng * 16;
+      t.zf = tab.size();
+      tab.resize(t.zf + (size_t)n * t.zf_ld, 0.0);
+      z_split(n, nt, ng);
+      t.zi_ld = nt * ng * 16;
+      t.zi = tab.size();
+      tab.resize(t.zi + (size_t)up(2 * L, 8) * t.zi_ld, 0.0);
+      for (int l = 0; l < L; l++)
+         for (int z = 0, q = 0, q3 = 3 * n / 4; z < n; z++) {
+            const double c = co[q], s = co[q3];
+            if ((q += l) >= n) q -= n;
+            if ((q3 += l) >= n) q3 -= n;
+            tab[t.zf + (size_t)z * t.zf_ld + l] = c;
+            tab[t.zf + (size_t)z * t.zf_ld + L + l] = s;
+            tab[t.zi + (size_t)l * t.zi_ld + z] = c;
+            tab[t.zi + (size_t)(L + l) * t.zi_ld + z] = s;
+         }
+   }
+   for (int d = 0; d < 2; d++) {   // x, y: forward e^{+} [n][m], inverse e^{-} [2 m + 1][n/2 + 1]
+      const int n = g.n[d], m = g.m[d];
+      const std::vector<double> co = roots(n);
+      t.f_ld[d] = up(m + 1, 16);
+      t.fr[d] = tab.size();
+      trig_table(tab, co, n, n, t.f_ld[d], 0, n, m + 1, false, 1.0);
+      t.fi[d] = tab.size();
+      trig_table(tab, co, n, n, t.f_ld[d], 0, n, m + 1, true, 1.0);
+      t.i_ld[d] = up(n / 2 + 1, 16);
+      const int kr = up(2 * m + 1, 4);
+      t.ir[d] = tab.size();
+      trig_table(tab, co, n, kr, t.i_ld[d], -m, 2 * m + 1, n / 2 + 1, false, 1.0);
+      t.ii[d] = tab.size();
+      trig_table(tab, co, n, kr, t.i_ld[d], -m, 2 * m + 1, n / 2 + 1, true, -1.0);
+   }
+   t.dec = tab.size();
+   tab.insert(tab.end(), dec.begin(), dec.end());
+   t.poly = tab.size();
+   static const std::vector<double> poly = window_polys<R>();   // the window's, the same for every grid
+   tab.insert(tab.end(), poly.begin(), poly.end());
+   t.data = std::move(tab);
+}
+}  // namespace
+
+void mgpu::grid_tables(const GridGeom &g, GridTables &t) {
+   if (g.fp64) build_tables<double>(g, t);
+   else build_tables<float>(g, t);
+}
+
+void mgpu::grid_rowmap(const GridGeom &g, const std::vector<KRow> &rows, std::vector<int> &map) {
+   map.assign((size_t)(g.m[0] + 1) * (2 * g.m[1] + 1), -1);
+   for (size_t r = 0; r < rows.size(); r++) map[(size_t)rows[r].h * (2 * g.m[1] + 1) + rows[r].k + g.m[1]] = (int)r;
+}
+
+namespace {
+template <class RI, class RO, int NT>
+void gz_launch(std::vector<LaunchRec> *rec, hipStream_t st, unsigned grid, const GzArgs &a, const RI *in,
+               const double *tab, RO *out) {
+   glaunch<k_gz<RI, RO, NT>, b_gz<RI, RO, NT>, 256>(rec, st, grid, 256, 0, a, in, tab, out);
+}
+
+template <class RI, class RO>
+void z_pass(std::vector<LaunchRec> *rec, hipStream_t st, int nlines, int K, int ncols, int ldt, const RI *in,
+            const double *tab, RO *out) {
+   GzArgs a;
+   int nt;
+   a.nlines = nlines; a.K = K; a.lda = K; a.ncols = ncols; a.ldt = ldt; a.ldo = ncols;
+   z_split(ncols, nt, a.ngrp);
+   a.nmt = (nlines + 15) / 16;
+   const unsigned grid = (a.nmt * a.ngrp + 3) / 4;
+   switch (nt) {
+   case 1: gz_launch<RI, RO, 1>(rec, st, grid, a, in, tab, out); break;
+   case 2: gz_launch<RI, RO, 2>(rec, st, grid, a, in, tab, out); break;
+   case 3: gz_launch<RI, RO, 3>(rec, st, grid, a, in, tab, out); break;
+   case 4: gz_launch<RI, RO, 4>(rec, st, grid, a, in, tab, out); break;
+   default: gz_launch<RI, RO, 5>(rec, st, grid, a, in, tab, out); break;
+   }
+}
+
+void c_pass(std::vector<LaunchRec> *rec, hipStream_t st, GcArgs a, const double *in, const double *er,
+            const double *ei, double *out) {
+   a.nmt = (a.M + 15) / 16;
+   a.nct = (a.N + 15) / 16;
+   const unsigned grid = (unsigned)(((long)a.nbatch * a.nmt * a.nct + 3) / 4);
+   glaunch<k_gc, b_gc, 256>(rec, st, grid, 256, 0, a, in, er, ei, out);
+}
+
+template <class R>
+void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const GridTables &t, const GridBufs &b,
+          bool join) {
+   const GridSizes z = grid_sizes(g);
+   hipStream_t st = e->stream;
+   uint8_t *B = b.base;
+   const double *tab = b.tab;
+   const double *poly = tab + t.poly;
+   const int ns = g.ns, nbr = g.nb[0] * g.nb[1] * g.nb[2];
+   const size_t L = g.m[2] + 1, P = (2 * g.m[1] + 1) * L;
+   int4 *anc = (int4 *)(B + z.anc);
+   int *cnt = (int *)(B + z.cnt), *start = (int *)(B + z.start);
+   R *G = (R *)(B + z.G);
+   double *T1 = (double *)(B + z.T1), *T2 = (double *)(B + z.T2), *T3 = (double *)(B + z.T3);
+   {
+      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_spread");
+      GBinArgs a;
+      for (int i = 0; i < 9; i++) a.hinv[i] = g.hinv[i];
+      for (int d = 0; d < 3; d++) { a.n[d] = g.n[d]; a.nb[d] = g.nb[d]; }
+      a.ns = ns; a.nsp = g.nsp; a.w = g.w; a.cap = g.cap;
+      a.site = b.site; a.sa = (int4 *)(B + z.sa); a.sx = (double *)(B + z.sx); a.cnt = cnt; a.bucket = (int *)(B + z.bucket);
+      glaunch<k_g_bin, b_g_bin, 256>(rec, st, (ns + 255) / 256, 256, 0, a);
+      glaunch<k_g_scan, b_g_scan, 256>(rec, st, 1, 256, 0, nbr, cnt, start);
+      GWtArgs w;
+      w.nb = nbr; w.ns = ns; w.nsp = g.nsp; w.cap = g.cap;
+      w.sa = a.sa; w.sx = a.sx; w.chg = b.w; w.bucket = a.bucket; w.start = start; w.cnt = cnt;
+      w.poly = poly; w.wt = B + z.wt; w.anc = anc; w.fr = (double4 *)(B + z.fr);
+      glaunch<k_g_weights<R>, b_g_weights<R>, 256>(rec, st, (nbr + 3) / 4, 256, (size_t)g.cap * (16 * 8 + 4 * 4), w);
+      GSpArgs s;
+      for (int d = 0; d < 3; d++) { s.n[d] = g.n[d]; s.nb[d] = g.nb[d]; }
+      glaunch<k_g_spread<R>, b_g_spread<R>, 256>(rec, st, nbr, 256, 0, s, (const R *)w.wt, anc, start, G);
+   }
+   GcArgs c;
+   {
+      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_forward");
+      z_pass<R, double>(rec, st, g.n[0] * g.n[1], g.n[2], 2 * L, t.zf_ld, G, tab + t.zf, T1);
+      c.nbatch = g.n[0]; c.K = g.n[1]; c.M = g.m[1] + 1; c.N = L; c.ldt = t.f_ld[1];
+      c.off = c.qoff = g.m[1]; c.mq = g.m[1] + 1;
+      c.inb = (size_t)g.n[1] * 2 * L; c.ink = 2 * L; c.inc = L; c.outb = 2 * P; c.outm = L; c.outc = P;
+      c_pass(rec, st, c, T1, tab + t.fr[1], tab + t.fi[1], T2);
+      c.nbatch = 1; c.K = g.n[0]; c.M = g.m[0] + 1; c.N = P; c.ldt = t.f_ld[0];
+      c.off = c.qoff = g.m[0]; c.mq = g.m[0] + 1;
+      c.inb = 0; c.ink = 2 * P; c.inc = P; c.outb = 0; c.outm = 2 * P; c.outc = P;
+      c_pass(rec, st, c, T2, tab + t.fr[0], tab + t.fi[0], T3);
+   }
+   {
+      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_kspace");
+      GkArgs k;
+      k.hmax = g.m[0]; k.kmax = g.m[1]; k.lmax = g.m[2];
+      k.vol = g.vol; k.r4a = -1.0 / (4.0 * g.alpha * g.alpha); k.c2 = 2 * PI_D * g.hinv[8];
+      k.rows = b.rows; k.rowmap = b.rowmap;
+      const double *dec = tab + t.dec;
+      k.dx = dec + t.dec_off[0]; k.dy = dec + t.dec_off[1]; k.dz = dec + t.dec_off[2];
+      k.bpart = (double *)(B + z.bpart);
+      glaunch<k_gk, b_gk, 256>(rec, st, z.nred, 256, 0, k, T3);
+   }
+   {
+      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_inverse");
+      c.nbatch = 1; c.K = 2 * g.m[0] + 1; c.M = g.n[0] / 2 + 1; c.N = P; c.ldt = t.i_ld[0];
+      c.off = 0; c.qoff = g.n[0]; c.mq = g.n[0] / 2;
+      c.inb = 0; c.ink = 2 * P; c.inc = P; c.outb = 0; c.outm = 2 * P; c.outc = P;
+      c_pass(rec, st, c, T3, tab + t.ir[0], tab + t.ii[0], T2);
+      c.nbatch = g.n[0]; c.K = 2 * g.m[1] + 1; c.M = g.n[1] / 2 + 1; c.N = L; c.ldt = t.i_ld[1];
+      c.off = 0; c.qoff = g.n[1]; c.mq = g.n[1] / 2;
+      c.inb = 2 * P; c.ink = L; c.inc = P; c.outb = (size_t)g.n[1] * 2 * L; c.outm = 2 * L; c.outc = L;
+      c_pass(rec, st, c, T2, tab + t.ir[1], tab + t.ii[1], T1);
+      z_pass<double, R>(rec, st, g.n[0] * g.n[1], 2 * L, g.n[2], t.zi_ld, T1, tab + t.zi, G);
+   }
+   {
+      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_gather");
+      GGaArgs a;
+      for (int d = 0; d < 3; d++) {
+         a.n[d] = g.n[d];
+         // k = h a* + k b* + l c* as ewald.c:445-447 forms it: c* along z only (a
+         // barostat's h may be tilted from that by a little)
+         for (int q = 0; q < 3; q++) a.m[3 * d + q] = d == 2 && q < 2 ? 0.0 : 2.0 * g.n[d] * g.hinv[3 * d + q];
+      }
+      const int nblk = (ns + 4 * GA_SPW - 1) / (4 * GA_SPW);
+      a.ns = ns; a.per = (nblk + 7) / 8; a.nsp = g.nsp;
+      // straight into the forces when no other stream is adding to them
+      const bool direct = !(join && e->join_pending);
+      a.add = direct;
+      double *fout = (double *)(B + z.fout);
+      glaunch<k_g_gather<R>, b_g_gather<R>, 256>(rec, st, 8 * a.per, 256, 0, a, G, poly, anc, (const double4 *)(B + z.fr),
+                                                 direct ? b.force : fout);
+      if (!direct) {
+         join_side(e);
+         glaunch<k_g_add, b_g_add, 256>(rec, st, (ns + 255) / 256, 256, 0, ns, g.nsp, fout, b.force);
+      }
+   }
+}
+}  // namespace
+
+void mgpu::grid_pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const GridTables &t,
+                     const GridBufs &b, bool join) {
+   if (g.fp64) pass<double>(e, rec, g, t, b, join);
+   else pass<float>(e, rec, g, t, b, join);
+}
+
+void mgpu::grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base) {
+   const GridSizes z = grid_sizes(g);
+   zero_async(e, base + z.cnt, 4 * (size_t)g.nb[0] * g.nb[1] * g.nb[2]);
+   zero_async(e, base + z.wt, z.wt_bytes);
+}
+
+bool mgpu::run_ewald_grid(mgpu_engine *e) {
+   const bool fp64 = e->precision == MGPU_FP64;
+   const GridGeom g = grid_geom(e->nsites, e->nsp, e->hmax, e->kmax, e->lmax, e->h, e->hinv, host_det(e->h),
+                                e->alpha, e->k_cutoff, fp64);
+   if (!grid_applies(g, e->nsitesxf, e->nk, e->k_cutoff, e->rows)) return false;
+   const GridSizes z = grid_sizes(g);
+   // the plan: tables of the grid's sizes, the k set's row map, and the
+   // cleared parts of the scratch block
+   const int key[8] = {g.n[0], g.n[1], g.n[2], g.m[0], g.m[1], g.m[2], fp64, g.ns};
+   const bool same = e->grid_tab && memcmp(key, e->grid_key, sizeof key) == 0;
+   if (e->capturing && (!same || e->grid_version != e->geom_version))
+      throw StatusError{MGPU_E_STATE, "gridded Ewald plan changed during capture"};
+   if (!same) {
+      auto t = std::make_shared<GridTables>();
+      grid_tables(g, *t);
+      e->d_gtab.reserve(t->data.size());
+      HIPCHK(hipMemcpyAsync(e->d_gtab.p, t->data.data(), t->data.size() * sizeof(double), hipMemcpyHostToDevice, e->stream));
+      HIPCHK(hipStreamSynchronize(e->stream));
+      e->grid_tab = t;
+      memcpy(e->grid_key, key, sizeof key);
+   }
+   if (e->d_grid.reserve(z.bytes) || !same) grid_clear(e, g, e->d_grid.p);
+   if (!same || e->grid_version != e->geom_version) {
+      std::vector<int> map;
+      grid_rowmap(g, e->rows, map);
+      e->d_growmap.reserve(map.size());
+      HIPCHK(hipMemcpyAsync(e->d_growmap.p, map.data(), sizeof(int) * map.size(), hipMemcpyHostToDevice, e->stream));
+      HIPCHK(hipStreamSynchronize(e->stream));
+      e->grid_version = e->geom_version;
+   }
+   e->d_out.reserve(OUT_SIZE);
+   GridBufs b;
+   b.site = e->d_site.p; b.w = e->d_chg_site.p; b.force = e->d_force_site.p;
+   b.rows = e->d_rows.p; b.rowmap = e->d_growmap.p; b.tab = e->d_gtab.p; b.base = e->d_grid.p; b.prof = true;
+   grid_pass(e, e->rec, g, *e->grid_tab, b, true);
+   const double *bpart = (const double *)(e->d_grid.p + z.bpart);
+   if (e->defer_recip) {   // the glue adds them (eval_forces_device)
+      e->recip_part = bpart;
+      e->recip_rows = z.nred;
+   } else {
+      reduce_cols(e, bpart, z.nred, 8, e->d_out.p + OUT_RECIP);
+   }
+   return true;
+}

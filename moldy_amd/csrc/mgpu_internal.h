@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 #include <map>
+#include <memory>
 
 #include "../../include/moldy_amd.h"
 #include "mgpu_group.h"
@@ -74,6 +75,10 @@ struct KRow {
 };
 
 }  // namespace mgpu
+
+namespace mgpu {
+struct GridTables;   // mgpu_ewald_grid.h
+}
 
 struct mgpu_engine {
    int device = 0;
@@ -201,6 +206,15 @@ struct mgpu_engine {
    std::vector<int> fwd_pos, fwd_tile_nb;       // each k row's forward position; per tile: blocks of 16 l
    int bp_version = -1;
 
+   // ---- gridded ewald: tables of the grid's sizes (key: grid points, largest
+   // |h| |k| |l|, FP64, sites), the k set's row map, scratch
+   std::shared_ptr<const mgpu::GridTables> grid_tab;
+   int grid_key[8] = {0};
+   int grid_version = -1;
+   mgpu::DBuf<double> d_gtab;
+   mgpu::DBuf<uint8_t> d_grid;
+   mgpu::DBuf<int> d_growmap;
+
    // ---- plan caching: uploads of k-set/slice metadata happen when the
    // geometry version changes, so a steady-state evaluation is launches only
    int geom_version = 0;
@@ -283,6 +297,7 @@ void run_pairlist_fill_device(mgpu_engine *e, int noff, long total);
 void run_rdf(mgpu_engine *e, double limit, int nbins, int noff, float *rdf_host);
 void run_ewald_fp64(mgpu_engine *e);        // -> d_out[OUT_RECIP..]
 void run_ewald_mixed(mgpu_engine *e);       // -> d_out[OUT_RECIP..]
+bool run_ewald_grid(mgpu_engine *e);        // the same; false (nothing done) where the direct sum is to run
 // The device part of eval_forces after the two boundary calls: second
 // make_sites, dipole and surface term, molecular forces and torques, virial
 // correction and the assembly of pe, dipole and stress into d_out[OUT_RES..].
