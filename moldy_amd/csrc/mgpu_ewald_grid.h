@@ -14,7 +14,7 @@ struct GridGeom {
 
 // Byte offsets into the scratch block.
 struct GridSizes {
-   size_t sa, sx, cnt, start, bucket, anc, fr, wt, wt_bytes, G, T1, T2, T3, bpart, fout, bytes;
+   size_t sa, sx, cnt, start, bucket, anc, fr, wt, G, T1, T2, T3, bpart, fout, bytes;
    int nred;                  // rows of bpart
 };
 
@@ -44,7 +44,7 @@ bool grid_pays(const GridGeom &g, int nk);
 GridSizes grid_sizes(const GridGeom &g);
 void grid_tables(const GridGeom &g, GridTables &t);
 void grid_rowmap(const GridGeom &g, const std::vector<KRow> &rows, std::vector<int> &map);
-// Clears what a pass expects cleared (brick counts, the weights' pads); a
+// Clears what a pass expects cleared (brick counts); a
 // pass leaves it so.
 void grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base);
 // The pass: per-block energy and stress sums at base + GridSizes::bpart

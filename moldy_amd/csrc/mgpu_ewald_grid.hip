@@ -58,9 +58,9 @@ template <> struct Win<float> {
    static constexpr int W = 8, DEG = 10;
    static constexpr double BETA = 2.6 * W;
 };
-// A site's spread weights: three rows of WP = W + 16, the W weights from
-// element 8 and zeros around them, so that a brick reads them at any offset.
-template <class R> constexpr int WP = Win<R>::W + 2 * GB;
+// A site's spread weights: three rows of W + 2, a zero at either end for every
+// grid point outside the window.
+template <class R> constexpr int WROW = Win<R>::W + 2;
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 // 16x16x4 matrix product: A row (B column) lane % 16 at k = lane / 16; item v
@@ -162,7 +162,7 @@ struct GWtArgs {
    const int *bucket, *start;
    int *cnt;             // cleared for the next pass
    const double *poly;   // [DEG + 1][W]
-   void *wt;             // R [ns][3][WP], pads already zero
+   void *wt;             // R [ns][3][W + 2]
    int4 *anc;            // brick order: anchor and site index
    double4 *fr;          // [ns]: arguments and charge
 };
@@ -172,7 +172,7 @@ struct GWtArgs {
 // than cap sites collects them by a walk over all sites.
 template <class R>
 __device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
-   constexpr int W = Win<R>::W, DEG = Win<R>::DEG, NL = 3 * W;
+   constexpr int W = Win<R>::W, DEG = Win<R>::DEG, WR = WROW<R>, NL = 3 * WR;
    extern __shared__ double gw_lds[];
    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
    const int b = bx * 4 + wave;
@@ -180,11 +180,11 @@ __device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
    double *xs = gw_lds + wave * 4 * a.cap;                  // the ranked sites' arguments and charges
    int *list = (int *)(gw_lds + 16 * a.cap) + wave * a.cap;
    const int m = a.cnt[b], s0 = a.start[b];
-   // lanes d * W + p: the polynomial of offset p on axis d
+   // lanes d WR + 1 + p: the polynomial of offset p on axis d
    double c[DEG + 1];
-   const int wd = lane / W, wp = lane % W;
+   const int wd = min(lane / WR, 2), wp = lane % WR - 1;
 #pragma unroll
-   for (int k = 0; k <= DEG; k++) c[k] = lane < NL ? a.poly[k * W + wp] : 0.0;
+   for (int k = 0; k <= DEG; k++) c[k] = lane < NL && wp >= 0 && wp < W ? a.poly[k * W + wp] : 0.0;
    auto place = [&](int i, int pos) {
       const int4 s = a.sa[i];
       a.anc[pos] = make_int4(s.x, s.y, s.z, i);
@@ -197,7 +197,7 @@ __device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
 #pragma unroll
       for (int k = DEG - 1; k >= 0; k--) v = v * x + c[k];
       if (wd == 0) v *= q;
-      if (lane < NL) ((R *)a.wt)[((size_t)pos * 3 + wd) * WP<R> + GB + wp] = (R)v;
+      if (lane < NL) ((R *)a.wt)[(size_t)pos * NL + lane] = (R)v;
    };
    if (m <= a.cap) {
       for (int t = lane; t < m; t += 64) list[t] = a.bucket[(size_t)b * a.cap + t];
@@ -213,7 +213,7 @@ __device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
          xs[4 * r + 3] = f.w;
       }
       wave_lds_sync();
-      for (int t = 0; t < m; t++) weights(xs[4 * t + min(wd, 2)], xs[4 * t + 3], s0 + t);
+      for (int t = 0; t < m; t++) weights(xs[4 * t + wd], xs[4 * t + 3], s0 + t);
    } else {
       int r = 0;
       for (int i0 = 0; i0 < a.ns; i0 += 64) {
@@ -223,7 +223,7 @@ __device__ __forceinline__ void b_g_weights(int bx, int nbx, const GWtArgs &a) {
          if (in) place(i, s0 + r + __popcll(mk & ((1ull << lane) - 1)));
          for (; mk; mk &= mk - 1, r++) {
             const int j = i0 + __builtin_ctzll(mk);
-            weights(a.sx[(size_t)min(wd, 2) * a.nsp + j], a.chg[j], s0 + r);
+            weights(a.sx[(size_t)wd * a.nsp + j], a.chg[j], s0 + r);
          }
       }
    }
@@ -236,69 +236,154 @@ template <class R> __global__ __launch_bounds__(256) void k_g_weights(GWtArgs a)
 // ------------------------------------------------------------ spread
 struct GSpArgs {
    int n[3], nb[3];
+   int ntz, per;         // z tiles of 16, blocks of each XCD
 };
 
-// One block per brick of 8^3 grid points; a lane holds the 8 points of one
-// (y, z) in registers.  The sites whose windows reach the brick have their
-// anchors in the W/8 + 1 (W = 16) or 2 (W = 8) bricks per axis up to it; the
-// four waves take every fourth of them.  A site's x weights are wave-uniform
-// (scalar loads), its y and z weights one load each, so a site costs a wave
-// about ten vector instructions for 512 points.
+typedef float flt4 __attribute__((ext_vector_type(4)));
+template <class R> struct SpM;
+template <> struct SpM<double> {
+   using V = dbl4;
+   static __device__ __forceinline__ V mul(double a, double b, V c) { return mma(a, b, c); }
+   static __device__ __forceinline__ int row(int g, int v) { return g + 4 * v; }
+};
+template <> struct SpM<float> {
+   using V = flt4;
+   static __device__ __forceinline__ V mul(float a, float b, V c) {
+      return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+   }
+   static __device__ __forceinline__ int row(int g, int v) { return 4 * g + v; }
+};
+
+// What bounds it: the matrix cores (the tiles of 8 x 8 x 16 multiply 4.5 times the
+// points the windows hold; 42% of their FP64 peak) and the operands' addresses.
+// 132,872 sites: 175 us FP64, 44 us FP32 (450 and 206 with one site a wave at a
+// time, its x weights as scalar loads: scalar issue bound it).
+// One block per tile of 8 x 8 x 16 grid points, as a product over the sites
+// whose windows reach it: rows (x, y) with q wx wy, columns z with wz, four
+// sites a step (lane / 16), four row tiles of 16.  Those sites have their
+// anchors in the 3 (W = 16) or 2 (W = 8) bricks per axis up to the tile's (one
+// more in z), each row of bricks along z one run of the brick-ordered sites, two
+// where it wraps; the four waves take every fourth group of four.  Weights are
+// read one group ahead.
 template <class R>
 __device__ __forceinline__ void b_g_spread(int bx, int nbx, const GSpArgs &a, const R *__restrict__ wt,
                                            const int4 *__restrict__ anc, const int *__restrict__ start,
                                            R *__restrict__ G) {
-   constexpr int W = Win<R>::W, P = WP<R>, NK = W > GB + 1 ? 3 : 2;
-   __shared__ R red[4][512];
+   constexpr int W = Win<R>::W, WR = WROW<R>, NK = W > GB + 1 ? 3 : 2, NR = NK * NK * 2;
+   using V = typename SpM<R>::V;
+   __shared__ R red[4][1024];
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-   const int ly = lane >> 3, lz = lane & 7;
+   const int m = lane & 15, g = lane >> 4;
    const int nby = a.nb[1], nbz = a.nb[2];
-   const int Bx = bx / (nby * nbz), By = bx / nbz - nby * Bx, Bz = bx - nbz * (By + nby * Bx);
-   const int zlo = Bz - (NK - 1);
-   R acc[GB];
-#pragma unroll
-   for (int r = 0; r < GB; r++) acc[r] = 0;
-   auto off = [](int base, int an, int n) {
-      int d = base - an;
-      if (d < -(GB - 1)) d += n;
-      return d + GB;
-   };
-   for (int ix = 0; ix < NK; ix++) {
-      const int cx = Bx - ix < 0 ? Bx - ix + a.nb[0] : Bx - ix;
-      for (int iy = 0; iy < NK; iy++) {
-         const int cy = By - iy < 0 ? By - iy + nby : By - iy;
-         const int cb = (cx * nby + cy) * nbz;
-         // the z run of bricks, in two pieces where it wraps
-         for (int pc = 0; pc < (zlo < 0 ? 2 : 1); pc++) {
-            const int z0 = pc == 0 ? max(zlo, 0) : zlo + nbz, z1 = pc == 0 ? Bz + 1 : nbz;
-            const int s = start[cb + z0], e = start[cb + z1];
-            int j = s + ((wave - s) & 3);
-            auto add = [&](const int4 A, int jj) {
-               const R *wr = wt + (size_t)jj * (3 * P);
-               const R *wx = wr + off(GB * Bx, A.x, a.n[0]);
-               const R wy = wr[P + off(GB * By, A.y, a.n[1]) + ly], wz = wr[2 * P + off(GB * Bz, A.z, a.n[2]) + lz];
-               const R t = wy * wz;
-#pragma unroll
-               for (int r = 0; r < GB; r++) acc[r] += wx[r] * t;
-            };
-            for (; j + 12 < e; j += 16) {
-               int4 A[4];
-#pragma unroll
-               for (int u = 0; u < 4; u++) A[u] = anc[j + 4 * u];
-#pragma unroll
-               for (int u = 0; u < 4; u++) add(A[u], j + 4 * u);
-            }
-            for (; j < e; j += 4) add(anc[j], j);
-         }
+   const int t = (bx & 7) * a.per + (bx >> 3);
+   if (t >= a.nb[0] * nby * a.ntz) return;   // block-uniform, before any barrier
+   const int Bx = t / (nby * a.ntz), By = t / a.ntz - nby * Bx, Tz = t - a.ntz * (By + nby * Bx);
+   // run r = (x brick, y brick, wrapped part): lane r holds its sites and its
+   // tile origin less the image shift, per axis
+   int rs = 0, re = 0, ox = 0, oy = 0, oz = 0;
+   if (lane < NR) {
+      const int q = lane >> 1, wrap = lane & 1;
+      int cx = Bx - q / NK, cy = By - q % NK;
+      ox = GB * Bx;
+      oy = GB * By;
+      oz = 2 * GB * Tz;
+      if (cx < 0) {
+         cx += a.nb[0];
+         ox += a.n[0];
       }
+      if (cy < 0) {
+         cy += nby;
+         oy += a.n[1];
+      }
+      const int zlo = 2 * Tz - (NK - 1), zhi = min(2 * Tz + 2, nbz);   // bricks [zlo, zhi)
+      int z0 = max(zlo, 0), z1 = zhi;
+      if (wrap) {
+         z0 = zlo + nbz;
+         z1 = zlo < 0 ? nbz : z0;
+         oz += a.n[2];
+      }
+      const int cb = (cx * nby + cy) * nbz;
+      rs = z1 > z0 ? start[cb + z0] : 0;
+      re = z1 > z0 ? start[cb + z1] : 0;
    }
+   V acc[4];
 #pragma unroll
-   for (int r = 0; r < GB; r++) red[wave][r * 64 + lane] = acc[r];
-   __syncthreads();
-   for (int t = threadIdx.x; t < 512; t += 256) {
-      const int x = GB * Bx + (t >> 6), y = GB * By + ((t >> 3) & 7), z = GB * Bz + (t & 7);
-      G[((size_t)x * a.n[1] + y) * a.n[2] + z] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+   for (int c = 0; c < 4; c++) acc[c] = V{0, 0, 0, 0};
+   int r = -1, base = 0, end = 0, rx = 0, ry = 0, rz = 0;
+   auto next = [&]() {   // the wave's next group of sites; false past the last run
+      base += 16;
+      while (base >= end) {
+         if (++r == NR) return false;
+         base = __builtin_amdgcn_readlane(rs, r) + 4 * wave;
+         end = __builtin_amdgcn_readlane(re, r);
+      }
+      rx = __builtin_amdgcn_readlane(ox, r);
+      ry = __builtin_amdgcn_readlane(oy, r);
+      rz = __builtin_amdgcn_readlane(oz, r);
+      return true;
+   };
+   // a group's anchors are loaded two groups ahead, its weights one
+   struct Op {
+      R wx[4], wy, wz;
+   };
+   int4 A = make_int4(0, 0, 0, 0);
+   int jc = 0, px = 0, py = 0, pz = 0;
+   auto fetch_anchor = [&]() {
+      const int j = base + g;
+      jc = min(j, end - 1);                       // a group holds at least one site
+      px = rx + (m >> 3);
+      py = ry + (m & 7);
+      pz = j < end ? rz + m : -(1 << 20);          // off the window: no weight
+      A = anc[jc];
+   };
+   auto fetch = [&](Op &o) {
+      const R *w = wt + (size_t)jc * (3 * WR) + 1;
+      const int dx = px - A.x;
+      o.wy = w[WR + min(max(py - A.y, -1), W)];
+      o.wz = w[2 * WR + min(max(pz - A.z, -1), W)];
+#pragma unroll
+      for (int c = 0; c < 4; c++) o.wx[c] = w[min(max(dx + 2 * c, -1), W)];
+   };
+   bool have = next(), more = false;
+   Op P, Q;
+   if (have) {
+      fetch_anchor();
+      fetch(P);
+      more = next();
+      if (more) fetch_anchor();
    }
+   auto step = [&](const Op &o, Op &ahead) {
+      R av[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) av[c] = o.wx[c] * o.wy;
+      have = more;
+      if (have) {
+         fetch(ahead);
+         more = next();
+         if (more) fetch_anchor();
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int c = 0; c < 4; c++) acc[c] = SpM<R>::mul(av[c], o.wz, acc[c]);
+   };
+   while (have) {
+      step(P, Q);
+      if (!have) break;
+      step(Q, P);
+   }
+   // row of tile c: x = 2 c + row / 8, y = row % 8
+#pragma unroll
+   for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) red[wave][(16 * c + SpM<R>::row(g, v)) * 16 + m] = acc[c][v];
+   __syncthreads();
+   const int z = 2 * GB * Tz + m;
+   if (z < a.n[2])
+      for (int q = threadIdx.x >> 4; q < 64; q += 16) {
+         const int o = q * 16 + m;
+         const int x = GB * Bx + (q >> 3), y = GB * By + (q & 7);
+         G[((size_t)x * a.n[1] + y) * a.n[2] + z] = ((red[0][o] + red[1][o]) + red[2][o]) + red[3][o];
+      }
 }
 template <class R>
 __global__ __launch_bounds__(256) void k_g_spread(GSpArgs a, const R *__restrict__ wt, const int4 *__restrict__ anc,
@@ -329,15 +414,38 @@ __device__ __forceinline__ void b_gz(int bx, int nbx, const GzArgs &a, const RI 
    dbl4 acc[NT];
 #pragma unroll
    for (int c = 0; c < NT; c++) acc[c] = dbl4{0, 0, 0, 0};
-   for (int k0 = 0; k0 < a.K; k0 += 8) {
-      const int k = k0 + 2 * g;
-      const T2 av = *(const T2 *)(ap + min(k, a.K - 2));   // K is even
+   // operands one step ahead (past the end: the last step's again)
+   struct Op {
+      T2 a;
+      double b0[NT], b1[NT];
+   };
+   const int klast = (a.K + 7) / 8 * 8 - 8;
+   auto load = [&](Op &o, int k0) {
+      const int k = min(k0, klast) + 2 * g;
+      o.a = *(const T2 *)(ap + min(k, a.K - 2));   // K is even
       const double *tp = tab + (size_t)k * a.ldt + c0;
 #pragma unroll
       for (int c = 0; c < NT; c++) {
-         acc[c] = mma(av.x, tp[16 * c], acc[c]);
-         acc[c] = mma(av.y, tp[a.ldt + 16 * c], acc[c]);
+         o.b0[c] = tp[16 * c];
+         o.b1[c] = tp[a.ldt + 16 * c];
       }
+   };
+   auto step = [&](const Op &o) {
+#pragma unroll
+      for (int c = 0; c < NT; c++) {
+         acc[c] = mma(o.a.x, o.b0[c], acc[c]);
+         acc[c] = mma(o.a.y, o.b1[c], acc[c]);
+      }
+   };
+   Op p, q;
+   load(p, 0);
+   for (int k0 = 0; k0 <= klast; k0 += 16) {
+      load(q, k0 + 8);
+      __builtin_amdgcn_sched_barrier(0);
+      step(p);
+      load(p, k0 + 16);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 + 8 <= klast) step(q);
    }
 #pragma unroll
    for (int v = 0; v < 4; v++) {
@@ -375,14 +483,39 @@ __device__ __forceinline__ void b_gc(int bx, int nbx, const GcArgs &a, const dou
    const double *ip = in + b * a.inb + min(n, a.N - 1);
    const double *rp = er + mt * 16 + m, *xp = ei + mt * 16 + m;
    dbl4 rr{0, 0, 0, 0}, ii{0, 0, 0, 0}, ri{0, 0, 0, 0}, ir{0, 0, 0, 0};
-   for (int k0 = 0; k0 < a.K; k0 += 4) {
-      const int k = k0 + g, kc = min(k, a.K - 1);   // the table's rows past K are zero
-      const double br = ip[kc * a.ink], bi = ip[kc * a.ink + a.inc];
-      const double ar = rp[(size_t)k * a.ldt], ai = xp[(size_t)k * a.ldt];
-      rr = mma(ar, br, rr);
-      ii = mma(ai, bi, ii);
-      ri = mma(ar, bi, ri);
-      ir = mma(ai, br, ir);
+   // operands of eight k, one step ahead (past the end: the last step's again)
+   struct Op {
+      double br[2], bi[2], ar[2], ai[2];
+   };
+   const int klast = (a.K + 7) / 8 * 8 - 8;
+   auto load = [&](Op &o, int k0) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+         const int k = min(k0, klast) + 4 * u + g, kc = min(k, a.K - 1);   // the table's rows past K are zero
+         o.br[u] = ip[kc * a.ink];
+         o.bi[u] = ip[kc * a.ink + a.inc];
+         o.ar[u] = rp[(size_t)k * a.ldt];
+         o.ai[u] = xp[(size_t)k * a.ldt];
+      }
+   };
+   auto step = [&](const Op &o) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+         rr = mma(o.ar[u], o.br[u], rr);
+         ii = mma(o.ai[u], o.bi[u], ii);
+         ri = mma(o.ar[u], o.bi[u], ri);
+         ir = mma(o.ai[u], o.br[u], ir);
+      }
+   };
+   Op p, q;
+   load(p, 0);
+   for (int k0 = 0; k0 <= klast; k0 += 16) {
+      load(q, k0 + 8);
+      __builtin_amdgcn_sched_barrier(0);
+      step(p);
+      load(p, k0 + 16);
+      __builtin_amdgcn_sched_barrier(0);
+      if (k0 + 8 <= klast) step(q);
    }
    if (n >= a.N) return;
 #pragma unroll
@@ -474,35 +607,103 @@ __global__ __launch_bounds__(256) void k_gk(GkArgs a, double *__restrict__ T) {
 
 // ------------------------------------------------------------ gather
 struct GGaArgs {
-   int n[3];
-   int ns, per;          // sites; blocks of each XCD
+   int n[3], nb[3];
+   int ntz, per;         // z tiles, blocks of each XCD
    double m[9];          // force = q sum_d G_d m[d]: 2 n_d hinv[d]
    int nsp, add;         // add: accumulate into out
 };
-constexpr int GA_SPW = 4;   // sites a wave takes in turn
+// Anchors per tile: 8 x 8 x GaT::TZ; the grid points their windows meet are
+// staged in LDS, RX x RX rows of RZ (a power of two).
+template <class R> struct GaT;
+template <> struct GaT<double> {
+   static constexpr int TZ = 16, RX = 23, RZ = 32, NW = 16;
+};
+template <> struct GaT<float> {
+   static constexpr int TZ = 8, RX = 15, RZ = 16, NW = 4;
+};
 
-// One wave per site (4 in turn, brick order, so that neighbours share the
-// grid lines they read; consecutive blocks on one XCD).  A lane holds a
-// (y, z) of the window and walks x; the weights and their derivatives come
-// from one polynomial a lane through LDS.
+template <int CTRL> __device__ __forceinline__ double row_ror(double x) {
+   const long long b = __builtin_bit_cast(long long, x);
+   const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
+   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_value(double x, int lane) {
+   const long long b = __builtin_bit_cast(long long, x);
+   const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// Sums of x, y, z over the wave, in every lane: x and y share the halves of a
+// register, z the odd rows of 16, so that 7 steps do for 18.
+__device__ __forceinline__ void wave_sum3(double &x, double &y, double &z, int lane) {
+   const bool hi = lane & 32, odd = lane & 16;
+   const double u = (hi ? y : x) + __shfl_xor(hi ? x : y, 32, 64), v = z + __shfl_xor(z, 32, 64);
+   double t = (odd ? v : u) + __shfl_xor(odd ? u : v, 16, 64);
+   t += row_ror<0x128>(t);
+   t += row_ror<0x124>(t);
+   t += row_ror<0x122>(t);
+   t += row_ror<0x121>(t);
+   x = lane_value(t, 0);
+   y = lane_value(t, 32);
+   z = lane_value(t, 16);
+}
+
+// What bounds it: LDS reads in FP64 (32 KB a site) and the chain of one site
+// (polynomials, window, wave sum).  132,872 sites: 230 us FP64, 57 us FP32 (331 and 78
+// reading the grid from L2).
+// One block per tile of anchors: the tile's sites are one run of the
+// brick-ordered sites, and every grid point their windows meet is read once
+// into LDS (read per site, a site's window of 2 x 128-byte lines a row is 64 KB
+// from L2 in FP64, 8.7 GB at 132,872 sites).  A wave per site in turn: a lane
+// holds a (y, z) of the window and walks x; the weights and their derivatives
+// come from one polynomial a lane through LDS.  Rows are turned by W elements
+// (every second one in FP64, second four in FP32) so that the rows a wave reads
+// together lie on different banks.
 template <class R>
 __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, const R *__restrict__ G,
                                            const double *__restrict__ poly, const int4 *__restrict__ anc,
-                                           const double4 *__restrict__ fr, double *__restrict__ out) {
+                                           const double4 *__restrict__ fr, const int *__restrict__ start,
+                                           double *__restrict__ out) {
    constexpr int W = Win<R>::W, DEG = Win<R>::DEG, NL = 3 * W, LY = 64 / W, NJ = W / LY;
+   constexpr int TZ = GaT<R>::TZ, RX = GaT<R>::RX, RZ = GaT<R>::RZ, NW = GaT<R>::NW, YS = W == 16 ? 0 : 2;
    using T2 = typename Vec<R>::T2;
-   __shared__ T2 sv[4][NL];
+   __shared__ R sg[RX * RX * RZ];
+   __shared__ T2 sv[NW][NL];
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
    const int wd = lane / W, wp = lane % W;
-   const int blk = (bx & 7) * a.per + (bx >> 3);
+   const int t = (bx & 7) * a.per + (bx >> 3);
+   if (t >= a.nb[0] * a.nb[1] * a.ntz) return;   // block-uniform, before any barrier
+   const int Bx = t / (a.nb[1] * a.ntz), By = t / a.ntz - a.nb[1] * Bx, Tz = t - a.ntz * (By + a.nb[1] * Bx);
+   const int cb = (Bx * a.nb[1] + By) * a.nb[2];
+   const int s0 = start[cb + Tz * (TZ / GB)], s1 = start[cb + min((Tz + 1) * (TZ / GB), a.nb[2])];
+   if (s1 == s0) return;   // block-uniform
+   {
+      const int z = threadIdx.x % RZ;
+      int zz = TZ * Tz + z;
+      if (zz >= a.n[2]) zz -= a.n[2];
+      if (z < TZ + W - 1) {
+#pragma unroll
+         for (int u = 0; u < (RX * RX * RZ + 64 * NW - 1) / (64 * NW); u++) {
+            const int r = threadIdx.x / RZ + u * (64 * NW / RZ);
+            if (r >= RX * RX) break;
+            int xx = GB * Bx + r / RX, yy = GB * By + r % RX;
+            if (xx >= a.n[0]) xx -= a.n[0];
+            if (yy >= a.n[1]) yy -= a.n[1];
+            sg[r * RZ + ((z + W * (((r % RX) >> YS) & 1)) & (RZ - 1))] = G[((size_t)xx * a.n[1] + yy) * a.n[2] + zz];
+         }
+      }
+   }
    double c[DEG + 1];
 #pragma unroll
    for (int k = 0; k <= DEG; k++) c[k] = lane < NL ? poly[k * W + wp] : 0.0;
-   for (int q = 0; q < GA_SPW; q++) {
-      const int pos = (blk * 4 + wave) * GA_SPW + q;
-      if (pos >= a.ns) return;   // wave-uniform; no block barrier in this kernel
-      const int4 A = anc[pos];
-      const double4 f = fr[pos];
+   int4 An = anc[min(s0 + wave, s1 - 1)];
+   double4 fn = fr[min(s0 + wave, s1 - 1)];
+   __syncthreads();
+   for (int pos = s0 + wave; pos < s1; pos += NW) {   // wave-uniform
+      const int4 A = An;
+      const double4 f = fn;
+      An = anc[min(pos + NW, s1 - 1)];
+      fn = fr[min(pos + NW, s1 - 1)];
       const double x = wd == 0 ? f.x : wd == 1 ? f.y : f.z;
       double v = c[DEG], dv = 0;
 #pragma unroll
@@ -512,33 +713,28 @@ __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, co
       }
       wave_lds_sync();
       if (lane < NL) {
-         T2 t;
-         t.x = (R)v;
-         t.y = (R)dv;
-         sv[wave][lane] = t;
+         T2 w;
+         w.x = (R)v;
+         w.y = (R)dv;
+         sv[wave][lane] = w;
       }
       wave_lds_sync();
-      int zz = A.z + wp;
-      if (zz >= a.n[2]) zz -= a.n[2];
-      int o[NJ];
+      const int lx = A.x - GB * Bx, lz = A.z - TZ * Tz + wp;
+      const R *gp[NJ];
 #pragma unroll
       for (int j = 0; j < NJ; j++) {
-         int yy = A.y + j * LY + wd;
-         if (yy >= a.n[1]) yy -= a.n[1];
-         o[j] = yy * a.n[2] + zz;
+         const int y = A.y - GB * By + j * LY + wd;
+         gp[j] = sg + (lx * RX + y) * RZ + ((lz + W * ((y >> YS) & 1)) & (RZ - 1));
       }
       R a0[NJ], a1[NJ];
 #pragma unroll
       for (int j = 0; j < NJ; j++) a0[j] = a1[j] = 0;
 #pragma unroll
       for (int i = 0; i < W; i++) {
-         int xx = A.x + i;
-         if (xx >= a.n[0]) xx -= a.n[0];
-         const R *gp = G + (size_t)xx * a.n[1] * a.n[2];
          const T2 wx = sv[wave][i];
 #pragma unroll
          for (int j = 0; j < NJ; j++) {
-            const R gv = gp[o[j]];
+            const R gv = gp[j][i * RX * RZ];
             a0[j] += wx.x * gv;
             a1[j] += wx.y * gv;
          }
@@ -552,8 +748,8 @@ __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, co
          p0 += (double)wy.x * (double)a0[j];
       }
       const T2 wz = sv[wave][2 * W + wp];
-      const double gx = wave_sum(px * (double)wz.x), gy = wave_sum(py * (double)wz.x),
-                   gz = wave_sum(p0 * (double)wz.y);
+      double gx = px * (double)wz.x, gy = py * (double)wz.x, gz = p0 * (double)wz.y;
+      wave_sum3(gx, gy, gz, lane);
       if (lane < 3) {
          const double fc = f.w * (gx * a.m[lane] + gy * a.m[3 + lane] + gz * a.m[6 + lane]);
          double *op = out + (size_t)lane * a.nsp + A.w;
@@ -562,10 +758,13 @@ __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, co
    }
 }
 template <class R>
-__global__ __launch_bounds__(256) void k_g_gather(GGaArgs a, const R *__restrict__ G,
-                                                  const double *__restrict__ poly, const int4 *__restrict__ anc,
-                                                  const double4 *__restrict__ fr, double *__restrict__ out) {
-   b_g_gather<R>(blockIdx.x, gridDim.x, a, G, poly, anc, fr, out);
+__global__ __launch_bounds__(64 * GaT<R>::NW) void k_g_gather(GGaArgs a, const R *__restrict__ G,
+                                                              const double *__restrict__ poly,
+                                                              const int4 *__restrict__ anc,
+                                                              const double4 *__restrict__ fr,
+                                                              const int *__restrict__ start,
+                                                              double *__restrict__ out) {
+   b_g_gather<R>(blockIdx.x, gridDim.x, a, G, poly, anc, fr, start, out);
 }
 
 // force += the gathered forces, once the real-space pass has added its own.
@@ -702,18 +901,18 @@ bool mgpu::grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const st
 
 // Where the grid beats the direct sum: its thirteen launches and its small
 // transforms cost a floor that N_k N_s products must outweigh.  MD step, direct
-// against grid: FP64 water, 8,800 sites (5.4e7 products) 218 and 256 us, 16,384
-// (1.9e8) 346 and 298, 120,000 (1.0e10) 6,404 and 1,113; mixed, 16,384 sites 185
-// and 220 us, 24,000 silica sites (8.2e8) 270 and 266, 120,000 1,053 and 627.
+// against grid: FP64 5,184 silica sites (3.8e7 products) 190 and 183 us, 8,800 water
+// sites (5.4e7) 216 and 226, 16,384 (1.9e8) 344 and 256, 132,872 salt water (1.3e10)
+// 7,870 and 1,112; mixed 16,384 water sites 184 and 193 us, 12,288 silica sites
+// (2.2e8) 191 and 181, 32,000 water (7.2e8) 290 and 237, 132,872 1,336 and 635.
 bool mgpu::grid_pays(const GridGeom &g, int nk) {
    const double direct = (double)nk * g.ns;
-   return direct > (g.fp64 ? 1.2e8 : 6e8);
+   return direct > (g.fp64 ? 8e7 : 2e8);
 }
 
 GridSizes mgpu::grid_sizes(const GridGeom &g) {
    GridSizes z;
    const size_t rs = g.fp64 ? 8 : 4, ns = g.ns;
-   const int wp = g.w + 2 * GB;
    const size_t L = g.m[2] + 1, P = (2 * g.m[1] + 1) * L;
    const size_t nb = (size_t)g.nb[0] * g.nb[1] * g.nb[2];
    size_t off = 0;
@@ -729,8 +928,7 @@ GridSizes mgpu::grid_sizes(const GridGeom &g) {
    z.bucket = take(4 * nb * g.cap);
    z.anc = take(16 * ns);
    z.fr = take(32 * ns);
-   z.wt = take(3 * (size_t)wp * rs * ns);
-   z.wt_bytes = 3 * (size_t)wp * rs * ns;
+   z.wt = take(3 * (size_t)(g.w + 2) * rs * ns);
    z.G = take(rs * g.n[0] * g.n[1] * g.n[2]);
    z.T1 = take(8 * g.n[0] * g.n[1] * 2 * L);
    z.T2 = take(8 * g.n[0] * 2 * P);
@@ -791,7 +989,7 @@ template <class R> void build_tables(const GridGeom &g, GridTables &t) {
       t.fi[d] = tab.size();
       trig_table(tab, co, n, n, t.f_ld[d], 0, n, m + 1, true, 1.0);
       t.i_ld[d] = up(n / 2 + 1, 16);
-      const int kr = up(2 * m + 1, 4);
+      const int kr = up(2 * m + 1, 8);
       t.ir[d] = tab.size();
       trig_table(tab, co, n, kr, t.i_ld[d], -m, 2 * m + 1, n / 2 + 1, false, 1.0);
       t.ii[d] = tab.size();
@@ -879,7 +1077,9 @@ void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const 
       glaunch<k_g_weights<R>, b_g_weights<R>, 256>(rec, st, (nbr + 3) / 4, 256, (size_t)g.cap * (16 * 8 + 4 * 4), w);
       GSpArgs s;
       for (int d = 0; d < 3; d++) { s.n[d] = g.n[d]; s.nb[d] = g.nb[d]; }
-      glaunch<k_g_spread<R>, b_g_spread<R>, 256>(rec, st, nbr, 256, 0, s, (const R *)w.wt, anc, start, G);
+      s.ntz = (g.nb[2] + 1) / 2;
+      s.per = (g.nb[0] * g.nb[1] * s.ntz + 7) / 8;
+      glaunch<k_g_spread<R>, b_g_spread<R>, 256>(rec, st, 8 * s.per, 256, 0, s, (const R *)w.wt, anc, start, G);
    }
    GcArgs c;
    {
@@ -926,14 +1126,18 @@ void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const 
          // barostat's h may be tilted from that by a little)
          for (int q = 0; q < 3; q++) a.m[3 * d + q] = d == 2 && q < 2 ? 0.0 : 2.0 * g.n[d] * g.hinv[3 * d + q];
       }
-      const int nblk = (ns + 4 * GA_SPW - 1) / (4 * GA_SPW);
-      a.ns = ns; a.per = (nblk + 7) / 8; a.nsp = g.nsp;
+      for (int d = 0; d < 3; d++) a.nb[d] = g.nb[d];
+      constexpr int TB = GaT<R>::TZ / GB;
+      a.ntz = (g.nb[2] + TB - 1) / TB;
+      a.per = (g.nb[0] * g.nb[1] * a.ntz + 7) / 8;
+      a.nsp = g.nsp;
       // straight into the forces when no other stream is adding to them
       const bool direct = !(join && e->join_pending);
       a.add = direct;
       double *fout = (double *)(B + z.fout);
-      glaunch<k_g_gather<R>, b_g_gather<R>, 256>(rec, st, 8 * a.per, 256, 0, a, G, poly, anc, (const double4 *)(B + z.fr),
-                                                 direct ? b.force : fout);
+      glaunch<k_g_gather<R>, b_g_gather<R>, 64 * GaT<R>::NW>(rec, st, 8 * a.per, 64 * GaT<R>::NW, 0, a, G, poly, anc,
+                                                             (const double4 *)(B + z.fr), start,
+                                                             direct ? b.force : fout);
       if (!direct) {
          join_side(e);
          glaunch<k_g_add, b_g_add, 256>(rec, st, (ns + 255) / 256, 256, 0, ns, g.nsp, fout, b.force);
@@ -951,7 +1155,6 @@ void mgpu::grid_pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom
 void mgpu::grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base) {
    const GridSizes z = grid_sizes(g);
    zero_async(e, base + z.cnt, 4 * (size_t)g.nb[0] * g.nb[1] * g.nb[2]);
-   zero_async(e, base + z.wt, z.wt_bytes);
 }
 
 bool mgpu::run_ewald_grid(mgpu_engine *e) {
