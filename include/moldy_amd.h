@@ -81,11 +81,10 @@ int  mgpu_set_precision(mgpu_engine *eng, int precision);
  * ewald run one after the other on the CPU. */
 int  mgpu_set_overlap(mgpu_engine *eng, int on);
 
-/* Real-space kernel: 0 automatic (the load-balanced kernel when the grid
- * holds at least 16 of its waves per CU), 1 the per-offset walk, 2 the
- * load-balanced kernel (one wave per site over the shell's z-columns of
- * cells) wherever the shell splits into columns, else the walk; 3 as 2 with
- * every site's candidates assigned to their column runs by binary search,
+/* Real-space kernel: 0 automatic (the load-balanced kernel from one site a
+ * CU), 1 the per-offset walk, 2 the load-balanced kernel (a wave takes sites
+ * in turn, each over the shell's z-columns of cells) wherever the shell splits into columns, else the walk; 3 as 2 with
+ * the candidates assigned to their column runs in windows of 64 instead of 2048,
  * the path taken by sites with more than 2048 candidates; 4 the tiled
  * Newton-3 kernel (every pair once, as force.c:717-778: one block per
  * z-column of cells, half of the shell's columns staged in LDS, the force on

@@ -387,6 +387,32 @@ __device__ __forceinline__ float wave_sumf(float v) {
    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
    return v;
 }
+template <int CTRL> __device__ __forceinline__ double row_ror(double x) {
+   const long long b = __builtin_bit_cast(long long, x);
+   const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, false);
+   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
+   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double lane_value(double x, int lane) {
+   const long long b = __builtin_bit_cast(long long, x);
+   const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+// Sums of x, y, z over the wave, in every lane: x and y share the halves of a
+// register, z the odd rows of 16, so that 7 steps do for 18.
+__device__ __forceinline__ void wave_sum3(double &x, double &y, double &z, int lane) {
+   const bool hi = lane & 32, odd = lane & 16;
+   const double u = (hi ? y : x) + __shfl_xor(hi ? x : y, 32, 64), v = z + __shfl_xor(z, 32, 64);
+   double t = (odd ? v : u) + __shfl_xor(odd ? u : v, 16, 64);
+   t += row_ror<0x128>(t);
+   t += row_ror<0x124>(t);
+   t += row_ror<0x122>(t);
+   t += row_ror<0x121>(t);
+   x = lane_value(t, 0);
+   y = lane_value(t, 32);
+   z = lane_value(t, 16);
+}
+
 // Cell index along one axis, restating cellbin (src/force.c:426-446): the
 // 8*DBL_EPSILON edge clamp, floor((s+0.5)*n), and the reference's two error
 // conditions as flag bits.

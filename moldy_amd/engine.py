@@ -223,8 +223,9 @@ class ForceEngine:
 
     def set_realspace_mode(self, mode):
         """Real-space kernel: RS_AUTO, RS_WALK (per-offset walk),
-        RS_BALANCED (one wave per site over the shell's z-columns),
-        RS_BALANCED_SEARCH (the same, candidates placed by binary search) or
+        RS_BALANCED (waves over the sites, candidates from the shell's
+        z-columns), RS_BALANCED_SEARCH (the same, candidates placed in
+        windows of 64 instead of 2048) or
         RS_TILED (Newton-3: every pair once, one block per z-column of cells,
         half of the shell's columns staged in LDS)."""
         self._chk(lib().mgpu_set_realspace_mode(self.h_, int(mode)))
