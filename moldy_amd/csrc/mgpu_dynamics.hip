@@ -54,13 +54,18 @@ __device__ __forceinline__ void rot_substep(const double *rot, double *L, double
    qmul(q, rot, q);
 }
 
+// Element i of three values by selection: an array indexed by a variable is
+// put into LDS (64 KB a block of k_coords, which left two blocks a CU).
+__device__ __forceinline__ double pick3(const double *x, int i) { return i == 0 ? x[0] : i == 1 ? x[1] : x[2]; }
+
 // make_rot, src/leapfrog.c:193-208: rotation about a principal axis
 __device__ __forceinline__ void rot_axis(double step, int axis, const double *L, double rinertia, double *rot) {
    double s, c;
-   sincos(0.5 * step * rinertia * L[axis + 1], &s, &c);
+   sincos(0.5 * step * rinertia * pick3(L + 1, axis), &s, &c);
    rot[0] = c;
-   rot[1] = rot[2] = rot[3] = 0.0;
-   rot[axis + 1] = s;
+   rot[1] = axis == 0 ? s : 0.0;
+   rot[2] = axis == 1 ? s : 0.0;
+   rot[3] = axis == 2 ? s : 0.0;
 }
 
 // make_rot_amom, src/leapfrog.c:213-231: rotation about L
@@ -126,17 +131,17 @@ __device__ __forceinline__ void b_coords(int bx, int nbx, const CoordArgs &a, co
       if (a.variant_a) {
          const int ax = ph == 0 || ph == 4 ? 0 : (ph == 2 ? 2 : 1);
          const double w = ph == 2 ? 1.0 : 0.5;
-         rot_axis(w * stepdts, ax, L, S.rI[ax], rot);
+         rot_axis(w * stepdts, ax, L, pick3(S.rI, ax), rot);
          rot_substep(rot, L, q);
       } else {
          const int s = a.saxis, o1 = (s + 1) % 3, o2 = (s + 2) % 3;
          if (ph == 1) {
-            rot_axis(stepdts, s, L, S.rI[s] - S.rI[o2], rot);
+            rot_axis(stepdts, s, L, pick3(S.rI, s) - pick3(S.rI, o2), rot);
             rot_substep(rot, L, q);
-            rot_amom(stepdts, L, S.rI[o2], rot);
+            rot_amom(stepdts, L, pick3(S.rI, o2), rot);
             qmul(q, rot, q);
          } else {
-            rot_axis(0.5 * stepdts, o1, L, S.rI[o1] - S.rI[o2], rot);
+            rot_axis(0.5 * stepdts, o1, L, pick3(S.rI, o1) - pick3(S.rI, o2), rot);
             rot_substep(rot, L, q);
          }
       }
@@ -153,7 +158,7 @@ __device__ __forceinline__ void b_coords(int bx, int nbx, const CoordArgs &a, co
 #pragma unroll
    for (int k = 0; k < 4; k++) { quat[4 * iq + k] = q[k]; amom[4 * iq + k] = L[k]; }
 }
-__global__ void k_coords(CoordArgs a, const int *__restrict__ mol_spec, const int *__restrict__ mol_quat,
+__global__ __launch_bounds__(256) void k_coords(CoordArgs a, const int *__restrict__ mol_spec, const int *__restrict__ mol_quat,
                          const SpecDyn *__restrict__ sd, const double *__restrict__ scal,
                          const double *__restrict__ mom, double *__restrict__ cm, double *__restrict__ quat,
                          double *__restrict__ amom, int *__restrict__ flags) {
@@ -281,16 +286,27 @@ __global__ __launch_bounds__(256) void k_dyad_part(KeArgs a, const int *__restri
    b_dyad_part(blockIdx.x, gridDim.x, a, mol_spec, mom, part);
 }
 
-// Column sums of the partials into out[0 .. nc), one thread per column.
+// Column sums of the partials into out[0 .. nc), one block: 256 / nc threads a
+// column each add every such row in order, then those sums are added in
+// order.  (One thread a column took 25 to 48 us for 135 to 422 rows, a load's
+// latency each.)
 __device__ __forceinline__ void b_col_sum(int bx, int nbx, int nblocks, int nc, const double *__restrict__ part,
                                           double *__restrict__ out) {
-   int c = threadIdx.x;
-   if (c >= nc) return;
+   __shared__ double s[256];
+   const int per = 256 / nc, c = (int)threadIdx.x % nc, q = (int)threadIdx.x / nc;
    double t = 0.0;
-   for (int b = 0; b < nblocks; b++) t += part[(size_t)b * nc + c];
-   out[c] = t;
+   if (q < per)
+      for (int b = q; b < nblocks; b += per) t += part[(size_t)b * nc + c];
+   s[threadIdx.x] = t;
+   __syncthreads();
+   if ((int)threadIdx.x < nc) {
+      double u = 0.0;
+      for (int k = 0; k < per; k++) u += s[k * nc + threadIdx.x];
+      out[threadIdx.x] = u;
+   }
 }
-__global__ void k_col_sum(int nblocks, int nc, const double *__restrict__ part, double *__restrict__ out) {
+__global__ __launch_bounds__(256) void k_col_sum(int nblocks, int nc, const double *__restrict__ part,
+                                                 double *__restrict__ out) {
    b_col_sum(blockIdx.x, gridDim.x, nblocks, nc, part, out);
 }
 
@@ -522,14 +538,14 @@ void ke_sums(mgpu_engine *e) {
    const int nb = (e->nmols + 255) / 256, nc = 4 * e->nspecies;
    glaunch<k_ke_part, b_ke_part, 256>(e->rec, e->stream, nb, 256, 0, ke_args(e), e->d_mol_spec.p, e->d_mol_quat.p,
                                       e->d_mom.p, e->d_amom.p, e->d_red.p);
-   glaunch<k_col_sum, b_col_sum, 1024>(e->rec, e->stream, 1, 128, 0, nb, nc, e->d_red.p, e->d_scal.p + S_KE);
+   glaunch<k_col_sum, b_col_sum, 256>(e->rec, e->stream, 1, 256, 0, nb, nc, e->d_red.p, e->d_scal.p + S_KE);
 }
 
 void dyad_sums(mgpu_engine *e) {
    const int nb = (e->nmols + 255) / 256, nc = 6 * e->nspecies;
    glaunch<k_dyad_part, b_dyad_part, 256>(e->rec, e->stream, nb, 256, 0, ke_args(e), e->d_mol_spec.p, e->d_mom.p,
                                           e->d_red.p);
-   glaunch<k_col_sum, b_col_sum, 1024>(e->rec, e->stream, 1, 128, 0, nb, nc, e->d_red.p, e->d_scal.p + S_DY);
+   glaunch<k_col_sum, b_col_sum, 256>(e->rec, e->stream, 1, 256, 0, nb, nc, e->d_red.p, e->d_scal.p + S_DY);
 }
 
 // One leapf_all_coords half step, with the thermostat's rotational terms
@@ -552,7 +568,7 @@ void coords_half(mgpu_engine *e) {
       c.ph_lo = lo;
       c.ph_hi = hi;
       c.normalise = hi == nph;
-      glaunch<k_coords, b_coords, 1024>(e->rec, e->stream, nb, 256, 0, c, e->d_mol_spec.p, e->d_mol_quat.p,
+      glaunch<k_coords, b_coords, 256>(e->rec, e->stream, nb, 256, 0, c, e->d_mol_spec.p, e->d_mol_quat.p,
                                         (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p, e->d_mom.p, e->d_cm.p,
                                         e->d_quat.p, e->d_amom.p, e->d_iflags.p);
    };
