@@ -132,7 +132,7 @@ void capture_batch(mgpu_batch *b) {
          mgpu_engine *e = b->eng[r];
          HIPCHK(hipStreamWaitEvent(e->stream, b->ev[0], 0));
          e->capturing = true;
-         md_step_launch(e, false);
+         md_step_launch(e);
          e->capturing = false;
          HIPCHK(hipEventRecord(b->ev[2 + r], e->stream));
          HIPCHK(hipStreamWaitEvent(b->origin, b->ev[2 + r], 0));
@@ -176,7 +176,7 @@ std::vector<LaunchRec> record_step(mgpu_engine *e) {
    try {
       e->rec = &recs;
       e->capturing = true;   // no timing events
-      md_step_launch(e, false);
+      md_step_launch(e);
    } catch (...) {
       undo();
       throw;
@@ -186,7 +186,7 @@ std::vector<LaunchRec> record_step(mgpu_engine *e) {
    HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
    e->capturing = true;
    try {
-      md_step_launch(e, false);
+      md_step_launch(e);
    } catch (...) {
       undo();
       hipGraph_t g = nullptr;
@@ -354,18 +354,17 @@ void enqueue_steps(mgpu_batch *b, int nsteps, bool init_h0, int s) {
                                               ": FP64 Ewald and surface-dipole steps have no grouped launches"};
    for (auto *e : b->eng) {
       md_load_cell(e);
-      md_reset_record(e, nsteps);
+      md_reset_record(e, nsteps, init_h0);
       zero_async(e, e->d_iflags.p, sizeof(int) * 48);
    }
    if (nsteps <= 0) return;
-   // The first step runs eagerly (it makes every buffer and may set H_0)
-   // unless the schedule's captured step is current and H_0 is kept: then
-   // every step is a replay.
-   const bool replay_all = !init_h0 && ((s == MGPU_SCHED_GROUPED && !grouped_stale(b)) ||
-                                        (s == MGPU_SCHED_GRAPH && !graph_stale(b)));
+   // The first step runs eagerly (it makes every buffer) unless the
+   // schedule's captured step is current: then every step is a replay.
+   const bool replay_all =
+       (s == MGPU_SCHED_GROUPED && !grouped_stale(b)) || (s == MGPU_SCHED_GRAPH && !graph_stale(b));
    const int first = replay_all ? 0 : 1;
    if (!replay_all) {
-      for (auto *e : b->eng) md_step_launch(e, init_h0);
+      for (auto *e : b->eng) md_step_launch(e);
       if (nsteps == 1) return;
    }
    if (s == MGPU_SCHED_GROUPED) {
@@ -394,7 +393,7 @@ void enqueue_steps(mgpu_batch *b, int nsteps, bool init_h0, int s) {
          for (auto *e : b->eng) HIPCHK(hipGraphLaunch(e->graph_exec, e->stream));
    } else {
       for (int k = 1; k < nsteps; k++)
-         for (auto *e : b->eng) md_step_launch(e, false);
+         for (auto *e : b->eng) md_step_launch(e);
    }
 }
 

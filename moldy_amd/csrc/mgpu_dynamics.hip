@@ -28,9 +28,10 @@ constexpr double DMIN = 2.2250738585072014e-308;
 
 // d_scal slots: thermostat, record row, per-species KE sums (4 a species),
 // cell h and hmom (row-major), per-species momentum dyads (6 a species)
-enum { S_TS = 0, S_TSMOM = 1, S_H0 = 2, S_ROW = 3, S_KE = 8, S_H = 64, S_HMOM = 73, S_DY = 82 };
+// S_INIT: the next step sets H_0 (so that the step itself is the same captured graph)
+enum { S_TS = 0, S_TSMOM = 1, S_H0 = 2, S_ROW = 3, S_INIT = 4, S_KE = 8, S_H = 64, S_HMOM = 73, S_DY = 82 };
 constexpr int MAX_SPEC = 14;              // S_KE + 4 * MAX_SPEC <= S_H
-constexpr int SCAL_SIZE = 192;            // S_DY + 6 * MAX_SPEC <= SCAL_SIZE
+constexpr int SCAL_SIZE = MGPU_SCAL_SIZE;            // S_DY + 6 * MAX_SPEC <= SCAL_SIZE
 constexpr int TRACE_W = 8;                // ke_t, ke_r, pe0, pe1, ts, tsmom, H_0, det(h)
 
 struct SpecDyn {
@@ -447,7 +448,7 @@ __device__ __forceinline__ void b_scalar(int bx, int nbx, const ScalArgs &a, con
             if (spec_rdof[s] > 0) kr += ke_rot(a, sd, scal, s);
          const double pe0 = res[0], pe1 = res[1];
          const double vol = det3(scal + S_H);
-         if (a.init_h0) {
+         if (scal[S_INIT] != 0.0) {
             scal[S_H0] = (kt + kr) + (pe0 + pe1) + tsmom * tsmom / (2.0 * a.ttmass) + a.gkt * log(ts) +
                          0.5 / a.pmass * sum_sq9(scal + S_HMOM);
             if (a.const_pressure) scal[S_H0] += a.pressure * vol;
@@ -459,10 +460,14 @@ __device__ __forceinline__ void b_scalar(int bx, int nbx, const ScalArgs &a, con
             t[7] = vol;
          }
          scal[S_ROW] = row + 1;
+         scal[S_INIT] = 0.0;
          break;
       }
       case OP_TSMOM_PE: tsmom -= a.step * (res[0] + res[1] - scal[S_H0]); break;
-      case OP_RESET_ROW: scal[S_ROW] = 0.0; break;
+      case OP_RESET_ROW:
+         scal[S_ROW] = 0.0;
+         scal[S_INIT] = a.init_h0 ? 1.0 : 0.0;
+         break;
       case OP_GLEAP_CELL: {
          // gleap_cell, src/leapfrog.c:475-508, at step = a.step / 2
          const double st = 0.5 * a.step;
@@ -675,6 +680,7 @@ void mgpu::md_setup(mgpu_engine *e, const mgpu_dynamics *d) {
    const int nb = (e->nmols + 255) / 256;
    e->d_red.reserve((size_t)nb * 6 * MAX_SPEC + 64);
    e->have_dyn = true;
+   e->geom_version++;   // captured steps hold the integrator's arguments
 }
 
 void mgpu::md_set_scalars(mgpu_engine *e, const double thermo[3]) {
@@ -686,8 +692,10 @@ void mgpu::md_set_scalars(mgpu_engine *e, const double thermo[3]) {
       v[S_H + i] = e->h[i];
       v[S_HMOM + i] = e->hmom[i];
    }
-   HIPCHK(hipMemcpyAsync(e->d_scal.p, v, sizeof v, hipMemcpyHostToDevice, e->stream));
-   HIPCHK(hipStreamSynchronize(e->stream));
+   const double *src[1] = {v};
+   double *dst[1] = {e->d_scal.p};
+   const size_t n[1] = {SCAL_SIZE};
+   upload_pinned(e, PIN_SCAL, 1, src, dst, n);
    memcpy(e->cell_loaded, v + S_H, sizeof e->cell_loaded);
    e->cell_valid = true;
 }
@@ -717,24 +725,23 @@ void mgpu::md_fetch_cell(mgpu_engine *e, double h[9], double hmom[9]) {
    }
 }
 
-void mgpu::md_get_scalars(mgpu_engine *e, double thermo[3]) {
-   double v[4];
-   HIPCHK(hipMemcpyAsync(v, e->d_scal.p, sizeof v, hipMemcpyDeviceToHost, e->stream));
-   HIPCHK(hipStreamSynchronize(e->stream));
+void mgpu::md_thermo(const double v[4], double thermo[3]) {
    thermo[0] = v[S_TS];
    thermo[1] = v[S_TSMOM];
    thermo[2] = v[S_H0];
 }
 
-void mgpu::md_reset_record(mgpu_engine *e, int cap) {
+void mgpu::md_reset_record(mgpu_engine *e, int cap, bool init_h0) {
    e->d_trace.reserve((size_t)std::max(cap, 1) * TRACE_W);
-   e->trace_cap = cap;
-   scalar_op(e, scal_args(e, OP_RESET_ROW));
+   e->trace_cap = (int)(e->d_trace.n / TRACE_W);   // what a captured step may fill in a longer call
+   ScalArgs a = scal_args(e, OP_RESET_ROW);
+   a.init_h0 = init_h0;
+   scalar_op(e, a);
 }
 
 // do_step, src/accel.c:626-827, at constant h, enqueued on e->stream with
 // no host synchronisation.
-void mgpu::md_step_launch(mgpu_engine *e, bool init_h0) {
+void mgpu::md_step_launch(mgpu_engine *e) {
    const bool therm = e->dyn_const_temp;
    if (therm) scalar_op(e, scal_args(e, OP_THERM_IN));
    if (therm) {
@@ -745,9 +752,7 @@ void mgpu::md_step_launch(mgpu_engine *e, bool init_h0) {
    eval_forces_device(e, false);
    momenta_half(e, false);
    ke_sums(e);
-   ScalArgs r = scal_args(e, OP_RECORD);
-   r.init_h0 = init_h0;
-   scalar_op(e, r);
+   scalar_op(e, scal_args(e, OP_RECORD));
    momenta_half(e, true);
    if (therm) scalar_op(e, scal_args(e, OP_TSMOM_PE));
    if (therm) {
@@ -761,7 +766,7 @@ void mgpu::md_step_launch(mgpu_engine *e, bool init_h0) {
 // do_step with the barostat (const_pressure branches of src/accel.c:686-779).
 // The cell half step runs on the device; the host then reads h, rebuilds the
 // link cells and the k-vector set for it and enqueues the rest of the step.
-void mgpu::md_step_pressure(mgpu_engine *e, bool init_h0) {
+void mgpu::md_step_pressure(mgpu_engine *e) {
    const bool therm = e->dyn_const_temp;
    if (therm) scalar_op(e, scal_args(e, OP_THERM_IN));
    scalar_op(e, scal_args(e, OP_GLEAP_CELL));
@@ -778,9 +783,7 @@ void mgpu::md_step_pressure(mgpu_engine *e, bool init_h0) {
    eval_forces_device(e, false);
    momenta_half(e, false);
    ke_sums(e);
-   ScalArgs r = scal_args(e, OP_RECORD);
-   r.init_h0 = init_h0;
-   scalar_op(e, r);
+   scalar_op(e, scal_args(e, OP_RECORD));
    momenta_half(e, true);
    if (therm) scalar_op(e, scal_args(e, OP_TSMOM_PE));
    scalar_op(e, scal_args(e, OP_HMOM_VIR));

@@ -1151,6 +1151,8 @@ bool mgpu::run_ewald_grid(mgpu_engine *e) {
       HIPCHK(hipStreamSynchronize(e->stream));
       e->grid_tab = t;
       memcpy(e->grid_key, key, sizeof key);
+      // a step captured with the old tables (another precision's, say) is stale
+      e->geom_version++;
    }
    if (e->d_grid.reserve(z.bytes) || !same) grid_clear(e, g, e->d_grid.p);
    if (!same || e->grid_version != e->geom_version) {

@@ -60,6 +60,18 @@ template <class T> struct DBuf {
    }
 };
 
+// Pinned host memory between the caller's arrays and the device.  An upload
+// copies into its region (state, momenta, scalars: one allocation, so that
+// they do not wait for one another) and returns with the transfers enqueued;
+// the region is busy until its event.
+enum { PIN_STATE = 0, PIN_MOM, PIN_SCAL, PIN_REGIONS };
+struct PinBuf {
+   double *p = nullptr;
+   size_t n = 0;
+   hipEvent_t ev[PIN_REGIONS] = {};
+   bool busy[PIN_REGIONS] = {};
+};
+
 // Per-kernel event timing (HIP events on the engine stream).
 struct KProf {
    double total_ms = 0;
@@ -109,6 +121,8 @@ struct mgpu_engine {
    bool intra_exact = false;   // every intramolecular pair is listed exactly once
    bool statics_done = false;
    int nsp = 0;        // padded site stride
+
+   mgpu::PinBuf pin_up, pin_down;               // host staging of the uploads and the downloads
 
    // ---- static device data ----
    mgpu::DBuf<int> d_site_type, d_site_mol, d_site_fw;
@@ -316,12 +330,19 @@ int adjoint_ntheta(const mgpu_engine *e);
 void run_adjoint(mgpu_engine *e, const double *v, const double *dtheta, double *dE, double *vjp, double *jvp);
 // molecular dynamics (mgpu_dynamics.hip)
 void md_setup(mgpu_engine *e, const mgpu_dynamics *d);
+// n[i] doubles from src[i] (host) to dst[i] (device) on e->stream through a
+// region of pin_up, for k arrays; src may be reused on return.
+void upload_pinned(mgpu_engine *e, int region, int k, const double *const *src, double *const *dst, const size_t *n);
+// n[i] doubles from src[i] (device) to dst[i] (host), complete on return.
+void download_pinned(mgpu_engine *e, int k, const double *const *src, double *const *dst, const size_t *n);
+#define MGPU_SCAL_SIZE 192   // integrator scalars (mgpu_dynamics.hip)
 void md_set_scalars(mgpu_engine *e, const double thermo[3]);
-void md_get_scalars(mgpu_engine *e, double thermo[3]);
-void md_reset_record(mgpu_engine *e, int cap);
-void md_step_launch(mgpu_engine *e, bool init_h0);
+void md_thermo(const double scal[4], double thermo[3]);   // from the first integrator scalars
+// A run of cap recorded steps; init_h0: its first step sets H_0.
+void md_reset_record(mgpu_engine *e, int cap, bool init_h0);
+void md_step_launch(mgpu_engine *e);
 void md_load_cell(mgpu_engine *e);
-void md_step_pressure(mgpu_engine *e, bool init_h0);
+void md_step_pressure(mgpu_engine *e);
 void md_fetch_cell(mgpu_engine *e, double h[9], double hmom[9]);
 void set_geometry(mgpu_engine *e, const double h[9]);
 // Size of the static device scratch array of mgpu_ewald_noalloc.
@@ -346,6 +367,7 @@ struct KSet {
 void build_kset(const double h[9], const double hinv[9], double kc, KSet &ks);
 // Main stream waits for the side stream's real-space pass (if one is pending).
 void join_side(mgpu_engine *e);
+bool step_graph_current(const mgpu_engine *e);
 void ensure_step_graph(mgpu_engine *e);
 void autotune_engine(mgpu_engine *e, int reps, int *sk_blocks, int *npart);
 void handle_flags(mgpu_engine *e, const int *fl);   // throws on error flags
