@@ -1085,6 +1085,7 @@ __global__ void k_jvp_phi(int ns, int nsp, const int *__restrict__ stype, const 
 
 // sum_i w_i exp(i k.r_i) for every k into cs[nk]
 static void weighted_sf(mgpu_engine *e, const double *w, double2 *cs) {
+   if (grid_weighted_sf(e, w, cs)) return;
    ewald_tables(e, w);
    const int nchunks = sfac_partials(e, e->nsites);
    k_sf_sum<<<(e->nk + 255) / 256, 256, 0, e->stream>>>(e->nk, nchunks, e->d_sk.p, cs);
@@ -1092,6 +1093,7 @@ static void weighted_sf(mgpu_engine *e, const double *w, double2 *cs) {
 
 // out[3][nsp] += w_i sum_k coeff k (C sin_i - S cos_i) with (C, S) = cs
 static void backproject(mgpu_engine *e, const double *w, const double4 *kc, const double2 *cs, double *out) {
+   if (grid_backproject(e, w, kc, cs, out)) return;
    e->d_wk.reserve((size_t)e->nk * 4 + 4);
    k_weights_w<<<(e->nk + 255) / 256, 256, 0, e->stream>>>(e->nk, kc, cs, e->d_wk.p);
    ewald_tables(e, w);

@@ -51,5 +51,10 @@ void grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base);
 // ([nred][8]), forces into b.force (after join_side when asked).
 void grid_pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const GridTables &t, const GridBufs &b,
                bool join);
+// For the charge adjoint of an FP64 engine: cs[k] = sum_i w_i exp(i k.r_i), and
+// out[3][nsp] += w_i sum_k coeff k (C sin_i - S cos_i) with (C, S) = cs and coeff
+// kc[k].w; false (nothing done) where the direct sum is to run.
+bool grid_weighted_sf(mgpu_engine *e, const double *w, double2 *cs);
+bool grid_backproject(mgpu_engine *e, const double *w, const double4 *kc, const double2 *cs, double *out);
 
 }  // namespace mgpu

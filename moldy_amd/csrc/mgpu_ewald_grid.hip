@@ -1021,43 +1021,67 @@ void c_pass(std::vector<LaunchRec> *rec, hipStream_t st, GcArgs a, const double 
    glaunch<k_gc, b_gc, 256>(rec, st, grid, 256, 0, a, in, er, ei, out);
 }
 
-template <class R>
-void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const GridTables &t, const GridBufs &b,
-          bool join) {
-   const GridSizes z = grid_sizes(g);
-   hipStream_t st = e->stream;
-   uint8_t *B = b.base;
-   const double *tab = b.tab;
-   const double *poly = tab + t.poly;
-   const int ns = g.ns, nbr = g.nb[0] * g.nb[1] * g.nb[2];
-   const size_t L = g.m[2] + 1, P = (2 * g.m[1] + 1) * L;
-   int4 *anc = (int4 *)(B + z.anc);
-   int *cnt = (int *)(B + z.cnt), *start = (int *)(B + z.start);
-   R *G = (R *)(B + z.G);
-   double *T1 = (double *)(B + z.T1), *T2 = (double *)(B + z.T2), *T3 = (double *)(B + z.T3);
-   {
-      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_spread");
+// The stages of a pass on explicit storage.
+template <class R> struct Stages {
+   mgpu_engine *e;
+   std::vector<LaunchRec> *rec;
+   const GridGeom &g;
+   const GridTables &t;
+   const GridBufs &b;
+   const GridSizes z;
+   const double *tab, *poly;
+   size_t L, P;
+   int4 *anc;
+   int *cnt, *start;
+   R *G;
+   double *T1, *T2, *T3;
+
+   Stages(mgpu_engine *e_, std::vector<LaunchRec> *rec_, const GridGeom &g_, const GridTables &t_, const GridBufs &b_)
+       : e(e_), rec(rec_), g(g_), t(t_), b(b_), z(grid_sizes(g_)), tab(b_.tab), poly(b_.tab + t_.poly) {
+      uint8_t *B = b.base;
+      L = g.m[2] + 1;
+      P = (2 * g.m[1] + 1) * L;
+      anc = (int4 *)(B + z.anc);
+      cnt = (int *)(B + z.cnt);
+      start = (int *)(B + z.start);
+      G = (R *)(B + z.G);
+      T1 = (double *)(B + z.T1);
+      T2 = (double *)(B + z.T2);
+      T3 = (double *)(B + z.T3);
+   }
+
+   // the sites into bricks, with their spread weights times w
+   void sites(const double *w) {
+      hipStream_t st = e->stream;
+      const int nbr = g.nb[0] * g.nb[1] * g.nb[2];
+      uint8_t *B = b.base;
       GBinArgs a;
       for (int i = 0; i < 9; i++) a.hinv[i] = g.hinv[i];
       for (int d = 0; d < 3; d++) { a.n[d] = g.n[d]; a.nb[d] = g.nb[d]; }
-      a.ns = ns; a.nsp = g.nsp; a.w = g.w; a.cap = g.cap;
-      a.site = b.site; a.sa = (int4 *)(B + z.sa); a.sx = (double *)(B + z.sx); a.cnt = cnt; a.bucket = (int *)(B + z.bucket);
-      glaunch<k_g_bin, b_g_bin, 256>(rec, st, (ns + 255) / 256, 256, 0, a);
+      a.ns = g.ns; a.nsp = g.nsp; a.w = g.w; a.cap = g.cap;
+      a.site = b.site; a.sa = (int4 *)(B + z.sa); a.sx = (double *)(B + z.sx); a.cnt = cnt;
+      a.bucket = (int *)(B + z.bucket);
+      glaunch<k_g_bin, b_g_bin, 256>(rec, st, (g.ns + 255) / 256, 256, 0, a);
       glaunch<k_g_scan, b_g_scan, 256>(rec, st, 1, 256, 0, nbr, cnt, start);
-      GWtArgs w;
-      w.nb = nbr; w.ns = ns; w.nsp = g.nsp; w.cap = g.cap;
-      w.sa = a.sa; w.sx = a.sx; w.chg = b.w; w.bucket = a.bucket; w.start = start; w.cnt = cnt;
-      w.poly = poly; w.wt = B + z.wt; w.anc = anc; w.fr = (double4 *)(B + z.fr);
-      glaunch<k_g_weights<R>, b_g_weights<R>, 256>(rec, st, (nbr + 3) / 4, 256, (size_t)g.cap * (16 * 8 + 4 * 4), w);
+      GWtArgs q;
+      q.nb = nbr; q.ns = g.ns; q.nsp = g.nsp; q.cap = g.cap;
+      q.sa = a.sa; q.sx = a.sx; q.chg = w; q.bucket = a.bucket; q.start = start; q.cnt = cnt;
+      q.poly = poly; q.wt = B + z.wt; q.anc = anc; q.fr = (double4 *)(B + z.fr);
+      glaunch<k_g_weights<R>, b_g_weights<R>, 256>(rec, st, (nbr + 3) / 4, 256, (size_t)g.cap * (16 * 8 + 4 * 4), q);
+   }
+
+   void spread() {
       GSpArgs s;
       for (int d = 0; d < 3; d++) { s.n[d] = g.n[d]; s.nb[d] = g.nb[d]; }
       s.ntz = (g.nb[2] + 1) / 2;
       s.per = (g.nb[0] * g.nb[1] * s.ntz + 7) / 8;
-      glaunch<k_g_spread<R>, b_g_spread<R>, 256>(rec, st, 8 * s.per, 256, 0, s, (const R *)w.wt, anc, start, G);
+      glaunch<k_g_spread<R>, b_g_spread<R>, 256>(rec, e->stream, 8 * s.per, 256, 0, s, (const R *)(b.base + z.wt), anc,
+                                                 start, G);
    }
-   GcArgs c;
-   {
-      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_forward");
+
+   void forward() {
+      hipStream_t st = e->stream;
+      GcArgs c;
       z_pass<R, double>(rec, st, g.n[0] * g.n[1], g.n[2], 2 * L, t.zf_ld, G, tab + t.zf, T1);
       c.nbatch = g.n[0]; c.K = g.n[1]; c.M = g.m[1] + 1; c.N = L; c.ldt = t.f_ld[1];
       c.off = c.qoff = g.m[1]; c.mq = g.m[1] + 1;
@@ -1068,19 +1092,10 @@ void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const 
       c.inb = 0; c.ink = 2 * P; c.inc = P; c.outb = 0; c.outm = 2 * P; c.outc = P;
       c_pass(rec, st, c, T2, tab + t.fr[0], tab + t.fi[0], T3);
    }
-   {
-      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_kspace");
-      GkArgs k;
-      k.hmax = g.m[0]; k.kmax = g.m[1]; k.lmax = g.m[2];
-      k.vol = g.vol; k.r4a = -1.0 / (4.0 * g.alpha * g.alpha); k.c2 = 2 * PI_D * g.hinv[8];
-      k.rows = b.rows; k.rowmap = b.rowmap;
-      const double *dec = tab + t.dec;
-      k.dx = dec + t.dec_off[0]; k.dy = dec + t.dec_off[1]; k.dz = dec + t.dec_off[2];
-      k.bpart = (double *)(B + z.bpart);
-      glaunch<k_gk, b_gk, 256>(rec, st, z.nred, 256, 0, k, T3);
-   }
-   {
-      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_inverse");
+
+   void inverse() {
+      hipStream_t st = e->stream;
+      GcArgs c;
       c.nbatch = 1; c.K = 2 * g.m[0] + 1; c.M = g.n[0] / 2 + 1; c.N = P; c.ldt = t.i_ld[0];
       c.off = 0; c.qoff = g.n[0]; c.mq = g.n[0] / 2;
       c.inb = 0; c.ink = 2 * P; c.inc = P; c.outb = 0; c.outm = 2 * P; c.outc = P;
@@ -1091,32 +1106,106 @@ void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const 
       c_pass(rec, st, c, T2, tab + t.ir[1], tab + t.ii[1], T1);
       z_pass<double, R>(rec, st, g.n[0] * g.n[1], 2 * L, g.n[2], t.zi_ld, T1, tab + t.zi, G);
    }
-   {
-      ProfScope ps(b.prof ? e : nullptr, "ewald_grid_gather");
+
+   void gather(double *out, bool add) {
       GGaArgs a;
       for (int d = 0; d < 3; d++) {
          a.n[d] = g.n[d];
+         a.nb[d] = g.nb[d];
          // k = h a* + k b* + l c* as ewald.c:445-447 forms it: c* along z only (a
          // barostat's h may be tilted from that by a little)
          for (int q = 0; q < 3; q++) a.m[3 * d + q] = d == 2 && q < 2 ? 0.0 : 2.0 * g.n[d] * g.hinv[3 * d + q];
       }
-      for (int d = 0; d < 3; d++) a.nb[d] = g.nb[d];
       constexpr int TB = GaT<R>::TZ / GB;
       a.ntz = (g.nb[2] + TB - 1) / TB;
       a.per = (g.nb[0] * g.nb[1] * a.ntz + 7) / 8;
       a.nsp = g.nsp;
+      a.add = add;
+      glaunch<k_g_gather<R>, b_g_gather<R>, 64 * GaT<R>::NW>(rec, e->stream, 8 * a.per, 64 * GaT<R>::NW, 0, a, G, poly,
+                                                             anc, (const double4 *)(b.base + z.fr), start, out);
+   }
+
+   const double *dec(int d) const { return tab + t.dec + t.dec_off[d]; }
+};
+
+template <class R>
+void pass(mgpu_engine *e, std::vector<LaunchRec> *rec, const GridGeom &g, const GridTables &t, const GridBufs &b,
+          bool join) {
+   Stages<R> s(e, rec, g, t, b);
+   mgpu_engine *pe = b.prof ? e : nullptr;
+   {
+      ProfScope ps(pe, "ewald_grid_spread");
+      s.sites(b.w);
+      s.spread();
+   }
+   {
+      ProfScope ps(pe, "ewald_grid_forward");
+      s.forward();
+   }
+   {
+      ProfScope ps(pe, "ewald_grid_kspace");
+      GkArgs k;
+      k.hmax = g.m[0]; k.kmax = g.m[1]; k.lmax = g.m[2];
+      k.vol = g.vol; k.r4a = -1.0 / (4.0 * g.alpha * g.alpha); k.c2 = 2 * PI_D * g.hinv[8];
+      k.rows = b.rows; k.rowmap = b.rowmap;
+      k.dx = s.dec(0); k.dy = s.dec(1); k.dz = s.dec(2);
+      k.bpart = (double *)(b.base + s.z.bpart);
+      glaunch<k_gk, b_gk, 256>(rec, e->stream, s.z.nred, 256, 0, k, s.T3);
+   }
+   {
+      ProfScope ps(pe, "ewald_grid_inverse");
+      s.inverse();
+   }
+   {
+      ProfScope ps(pe, "ewald_grid_gather");
       // straight into the forces when no other stream is adding to them
       const bool direct = !(join && e->join_pending);
-      a.add = direct;
-      double *fout = (double *)(B + z.fout);
-      glaunch<k_g_gather<R>, b_g_gather<R>, 64 * GaT<R>::NW>(rec, st, 8 * a.per, 64 * GaT<R>::NW, 0, a, G, poly, anc,
-                                                             (const double4 *)(B + z.fr), start,
-                                                             direct ? b.force : fout);
+      double *fout = (double *)(b.base + s.z.fout);
+      s.gather(direct ? b.force : fout, direct);
       if (!direct) {
          join_side(e);
-         glaunch<k_g_add, b_g_add, 256>(rec, st, (ns + 255) / 256, 256, 0, ns, g.nsp, fout, b.force);
+         glaunch<k_g_add, b_g_add, 256>(rec, e->stream, (g.ns + 255) / 256, 256, 0, g.ns, g.nsp, fout, b.force);
       }
    }
+}
+
+// Place of k vector k's mode in the dense box, and whether it is held as
+// its inverse (l < 0).
+struct GxArgs {
+   int nk, hmax, kmax, lmax;
+   const KRow *rows;
+   const int *krow;
+   const double *dx, *dy, *dz;
+};
+__device__ __forceinline__ size_t mode_of(const GxArgs &a, int k, bool &conj, double &dec) {
+   const KRow R = a.rows[a.krow[k]];
+   const int l = R.l0 + (k - R.kstart), L = a.lmax + 1, P = (2 * a.kmax + 1) * L;
+   conj = l < 0;
+   const int h = conj ? -R.h : R.h, kk = conj ? -R.k : R.k, ll = conj ? -l : l;
+   dec = a.dx[R.h] * a.dy[R.k < 0 ? -R.k : R.k] * a.dz[ll];
+   return (size_t)(h + a.hmax) * 2 * P + (kk + a.kmax) * L + ll;
+}
+// cs[k] = S(k) from the transformed grid.
+__global__ __launch_bounds__(256) void k_g_sf(GxArgs a, const double *__restrict__ T, double2 *__restrict__ cs) {
+   const int k = blockIdx.x * 256 + threadIdx.x;
+   if (k >= a.nk) return;
+   bool conj;
+   double dec;
+   const size_t o = mode_of(a, k, conj, dec);
+   const double s = dec * T[o + (2 * a.kmax + 1) * (a.lmax + 1)];
+   cs[k] = make_double2(dec * T[o], conj ? -s : s);
+}
+// The inverse transform's weights coeff S from cs, into a cleared T.
+__global__ __launch_bounds__(256) void k_g_fill(GxArgs a, const double4 *__restrict__ kc, const double2 *__restrict__ cs,
+                                                double *__restrict__ T) {
+   const int k = blockIdx.x * 256 + threadIdx.x;
+   if (k >= a.nk) return;
+   bool conj;
+   double dec;
+   const size_t o = mode_of(a, k, conj, dec);
+   const double w = dec * kc[k].w;
+   T[o] = w * cs[k].x;
+   T[o + (2 * a.kmax + 1) * (a.lmax + 1)] = conj ? -w * cs[k].y : w * cs[k].y;
 }
 }  // namespace
 
@@ -1131,9 +1220,11 @@ void mgpu::grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base) {
    zero_async(e, base + z.cnt, 4 * (size_t)g.nb[0] * g.nb[1] * g.nb[2]);
 }
 
-bool mgpu::run_ewald_grid(mgpu_engine *e) {
+// The engine's plan for its geometry and precision, made where it is missing
+// or stale; false where the direct sum is to run.
+static bool grid_plan(mgpu_engine *e, GridGeom &g) {
    const bool fp64 = e->precision == MGPU_FP64;
-   const GridGeom g = grid_geom(e->nsites, e->nsp, e->hmax, e->kmax, e->lmax, e->h, e->hinv, host_det(e->h),
+   g = grid_geom(e->nsites, e->nsp, e->hmax, e->kmax, e->lmax, e->h, e->hinv, host_det(e->h),
                                 e->alpha, e->k_cutoff, fp64);
    if (!grid_applies(g, e->nsitesxf, e->nk, e->k_cutoff, e->rows)) return false;
    const GridSizes z = grid_sizes(g);
@@ -1163,11 +1254,22 @@ bool mgpu::run_ewald_grid(mgpu_engine *e) {
       HIPCHK(hipStreamSynchronize(e->stream));
       e->grid_version = e->geom_version;
    }
-   e->d_out.reserve(OUT_SIZE);
+   return true;
+}
+
+static GridBufs grid_bufs(mgpu_engine *e) {
    GridBufs b;
    b.site = e->d_site.p; b.w = e->d_chg_site.p; b.force = e->d_force_site.p;
    b.rows = e->d_rows.p; b.rowmap = e->d_growmap.p; b.tab = e->d_gtab.p; b.base = e->d_grid.p; b.prof = true;
-   grid_pass(e, e->rec, g, *e->grid_tab, b, true);
+   return b;
+}
+
+bool mgpu::run_ewald_grid(mgpu_engine *e) {
+   GridGeom g;
+   if (!grid_plan(e, g)) return false;
+   const GridSizes z = grid_sizes(g);
+   e->d_out.reserve(OUT_SIZE);
+   grid_pass(e, e->rec, g, *e->grid_tab, grid_bufs(e), true);
    const double *bpart = (const double *)(e->d_grid.p + z.bpart);
    if (e->defer_recip) {   // the glue adds them (eval_forces_device)
       e->recip_part = bpart;
@@ -1175,5 +1277,34 @@ bool mgpu::run_ewald_grid(mgpu_engine *e) {
    } else {
       reduce_cols(e, bpart, z.nred, 8, e->d_out.p + OUT_RECIP);
    }
+   return true;
+}
+
+static GxArgs mode_args(mgpu_engine *e, const Stages<double> &s) {
+   return GxArgs{e->nk, s.g.m[0], s.g.m[1], s.g.m[2], e->d_rows.p, e->d_krow.p, s.dec(0), s.dec(1), s.dec(2)};
+}
+
+bool mgpu::grid_weighted_sf(mgpu_engine *e, const double *w, double2 *cs) {
+   GridGeom g;
+   if (e->precision != MGPU_FP64 || !grid_plan(e, g)) return false;
+   const GridBufs b = grid_bufs(e);
+   Stages<double> s(e, nullptr, g, *e->grid_tab, b);
+   s.sites(w);
+   s.spread();
+   s.forward();
+   k_g_sf<<<(e->nk + 255) / 256, 256, 0, e->stream>>>(mode_args(e, s), s.T3, cs);
+   return true;
+}
+
+bool mgpu::grid_backproject(mgpu_engine *e, const double *w, const double4 *kc, const double2 *cs, double *out) {
+   GridGeom g;
+   if (e->precision != MGPU_FP64 || !grid_plan(e, g)) return false;
+   const GridBufs b = grid_bufs(e);
+   Stages<double> s(e, nullptr, g, *e->grid_tab, b);
+   s.sites(w);
+   zero_async(e, s.T3, sizeof(double) * (2 * g.m[0] + 1) * 2 * s.P);
+   k_g_fill<<<(e->nk + 255) / 256, 256, 0, e->stream>>>(mode_args(e, s), kc, cs, s.T3);
+   s.inverse();
+   s.gather(out, true);
    return true;
 }
