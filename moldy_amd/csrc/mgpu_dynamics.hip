@@ -97,13 +97,10 @@ struct CoordArgs {
 // delta about o1, 1 precession about the symmetry axis and spin about L, 2
 // half delta about o1) or leapf_quat_a (leapfrog.c:345-392: axes 0,1,2,1,0
 // with weights 1/2,1/2,1,1/2,1/2), then normalise (leapfrog.c:96-113).
-__device__ __forceinline__ void b_coords(int bx, int nbx, const CoordArgs &a, const int *__restrict__ mol_spec,
-                                         const int *__restrict__ mol_quat, const SpecDyn *__restrict__ sd,
-                                         const double *__restrict__ scal, const double *__restrict__ mom,
-                                         double *__restrict__ cm, double *__restrict__ quat,
-                                         double *__restrict__ amom, int *__restrict__ flags) {
-   int m = bx * blockDim.x + threadIdx.x;
-   if (m >= a.nmols) return;
+// One molecule m (no restrict: the fused kernels write mom and amom first).
+__device__ __forceinline__ void coords_one(int m, const CoordArgs &a, const int *mol_spec, const int *mol_quat,
+                                           const SpecDyn *sd, const double *scal, const double *mom, double *cm,
+                                           double *quat, double *amom, int *flags) {
    const int sp = mol_spec[m];
    const SpecDyn S = sd[sp];
    const double ts = scal[S_TS];
@@ -159,6 +156,12 @@ __device__ __forceinline__ void b_coords(int bx, int nbx, const CoordArgs &a, co
 #pragma unroll
    for (int k = 0; k < 4; k++) { quat[4 * iq + k] = q[k]; amom[4 * iq + k] = L[k]; }
 }
+__device__ __forceinline__ void b_coords(int bx, int nbx, const CoordArgs &a, const int *mol_spec,
+                                         const int *mol_quat, const SpecDyn *sd, const double *scal,
+                                         const double *mom, double *cm, double *quat, double *amom, int *flags) {
+   const int m = bx * 256 + threadIdx.x;
+   if (m < a.nmols) coords_one(m, a, mol_spec, mol_quat, sd, scal, mom, cm, quat, amom, flags);
+}
 __global__ __launch_bounds__(256) void k_coords(CoordArgs a, const int *__restrict__ mol_spec, const int *__restrict__ mol_quat,
                          const SpecDyn *__restrict__ sd, const double *__restrict__ scal,
                          const double *__restrict__ mom, double *__restrict__ cm, double *__restrict__ quat,
@@ -174,13 +177,9 @@ struct MomArgs {
 };
 
 // leapf_all_momenta, src/accel.c:376-388 (leapf_mom, leapf_amom)
-__device__ __forceinline__ void b_momenta(int bx, int nbx, const MomArgs &a, const int *__restrict__ mol_spec,
-                                          const int *__restrict__ mol_quat, const SpecDyn *__restrict__ sd,
-                                          const double *__restrict__ scal, const double *__restrict__ force,
-                                          const double *__restrict__ torque, double *__restrict__ mom,
-                                          double *__restrict__ amom) {
-   int m = bx * blockDim.x + threadIdx.x;
-   if (m >= a.nmols) return;
+__device__ __forceinline__ void mom_one(int m, const MomArgs &a, const int *mol_spec, const int *mol_quat,
+                                        const SpecDyn *sd, const double *scal, const double *force,
+                                        const double *torque, double *mom, double *amom) {
    const double c = a.step * scal[S_TS];
    double A[9];
 #pragma unroll
@@ -199,11 +198,34 @@ __device__ __forceinline__ void b_momenta(int bx, int nbx, const MomArgs &a, con
       amom[4 * iq + 3] += c * torque[3 * iq + 2];
    }
 }
-__global__ void k_momenta(MomArgs a, const int *__restrict__ mol_spec, const int *__restrict__ mol_quat,
-                          const SpecDyn *__restrict__ sd, const double *__restrict__ scal,
-                          const double *__restrict__ force, const double *__restrict__ torque,
-                          double *__restrict__ mom, double *__restrict__ amom) {
+__device__ __forceinline__ void b_momenta(int bx, int nbx, const MomArgs &a, const int *mol_spec,
+                                          const int *mol_quat, const SpecDyn *sd, const double *scal,
+                                          const double *force, const double *torque, double *mom, double *amom) {
+   const int m = bx * 256 + threadIdx.x;
+   if (m < a.nmols) mom_one(m, a, mol_spec, mol_quat, sd, scal, force, torque, mom, amom);
+}
+__global__ __launch_bounds__(256) void k_momenta(MomArgs a, const int *mol_spec, const int *mol_quat,
+                                                 const SpecDyn *sd, const double *scal, const double *force,
+                                                 const double *torque, double *mom, double *amom) {
    b_momenta(blockIdx.x, gridDim.x, a, mol_spec, mol_quat, sd, scal, force, torque, mom, amom);
+}
+
+// The second momentum half step and, without a thermostat's scalars between
+// them, the coordinate half step after it: one launch for two.
+__device__ __forceinline__ void b_mom_coords(int bx, int nbx, const MomArgs &a, const CoordArgs &c,
+                                             const int *mol_spec, const int *mol_quat, const SpecDyn *sd,
+                                             const double *scal, const double *force, const double *torque,
+                                             double *mom, double *cm, double *quat, double *amom, int *flags) {
+   const int m = bx * 256 + threadIdx.x;
+   if (m >= a.nmols) return;
+   mom_one(m, a, mol_spec, mol_quat, sd, scal, force, torque, mom, amom);
+   coords_one(m, c, mol_spec, mol_quat, sd, scal, mom, cm, quat, amom, flags);
+}
+__global__ __launch_bounds__(256) void k_mom_coords(MomArgs a, CoordArgs c, const int *mol_spec, const int *mol_quat,
+                                                    const SpecDyn *sd, const double *scal, const double *force,
+                                                    const double *torque, double *mom, double *cm, double *quat,
+                                                    double *amom, int *flags) {
+   b_mom_coords(blockIdx.x, gridDim.x, a, c, mol_spec, mol_quat, sd, scal, force, torque, mom, cm, quat, amom, flags);
 }
 
 struct KeArgs {
@@ -214,9 +236,8 @@ struct KeArgs {
 // Per-species sums of |p_real|^2 and amom_k^2 (k = 1..3): columns 4s+0..3
 // of a [nblocks][4 nspec] partial array (trans_ke and rot_ke numerators,
 // src/algorith.c:221-259).  Deterministic: wave sums, fixed block order.
-__device__ __forceinline__ void b_ke_part(int bx, int nbx, const KeArgs &a, const int *__restrict__ mol_spec,
-                                          const int *__restrict__ mol_quat, const double *__restrict__ mom,
-                                          const double *__restrict__ amom, double *__restrict__ part) {
+__device__ __forceinline__ void b_ke_part(int bx, int nbx, const KeArgs &a, const int *mol_spec,
+                                          const int *mol_quat, const double *mom, const double *amom, double *part) {
    __shared__ double ws[4][4 * MAX_SPEC];
    int m = bx * 256 + threadIdx.x;
    double v[4] = {0, 0, 0, 0};
@@ -251,6 +272,21 @@ __global__ __launch_bounds__(256) void k_ke_part(KeArgs a, const int *__restrict
                                                  const int *__restrict__ mol_quat, const double *__restrict__ mom,
                                                  const double *__restrict__ amom, double *__restrict__ part) {
    b_ke_part(blockIdx.x, gridDim.x, a, mol_spec, mol_quat, mom, amom, part);
+}
+
+// The first momentum half step and the kinetic sums of what it leaves.
+__device__ __forceinline__ void b_mom_ke(int bx, int nbx, const MomArgs &a, const KeArgs &k, const int *mol_spec,
+                                         const int *mol_quat, const SpecDyn *sd, const double *scal,
+                                         const double *force, const double *torque, double *mom, double *amom,
+                                         double *part) {
+   const int m = bx * 256 + threadIdx.x;
+   if (m < a.nmols) mom_one(m, a, mol_spec, mol_quat, sd, scal, force, torque, mom, amom);
+   b_ke_part(bx, nbx, k, mol_spec, mol_quat, mom, amom, part);   // each thread its own molecule again
+}
+__global__ __launch_bounds__(256) void k_mom_ke(MomArgs a, KeArgs k, const int *mol_spec, const int *mol_quat,
+                                                const SpecDyn *sd, const double *scal, const double *force,
+                                                const double *torque, double *mom, double *amom, double *part) {
+   b_mom_ke(blockIdx.x, gridDim.x, a, k, mol_spec, mol_quat, sd, scal, force, torque, mom, amom, part);
 }
 
 // Per-species sums of the real-momentum dyad p p^T (energy_dyad,
@@ -291,8 +327,7 @@ __global__ __launch_bounds__(256) void k_dyad_part(KeArgs a, const int *__restri
 // column each add every such row in order, then those sums are added in
 // order.  (One thread a column took 25 to 48 us for 135 to 422 rows, a load's
 // latency each.)
-__device__ __forceinline__ void b_col_sum(int bx, int nbx, int nblocks, int nc, const double *__restrict__ part,
-                                          double *__restrict__ out) {
+__device__ __forceinline__ void b_col_sum(int bx, int nbx, int nblocks, int nc, const double *part, double *out) {
    __shared__ double s[256];
    const int per = 256 / nc, c = (int)threadIdx.x % nc, q = (int)threadIdx.x / nc;
    double t = 0.0;
@@ -327,6 +362,7 @@ enum {
 
 struct ScalArgs {
    int op, nspec, init_h0, trace_cap;
+   int ke_rows;          // rows of kinetic partials to sum into S_KE first (0: none)
    double step, ttmass, pmass, gkt;
    double w[3];                 // per-axis weights (OP_TSMOM_AXES), order of addition
    int axes[3], naxes;
@@ -413,10 +449,14 @@ __device__ double ke_rot(const ScalArgs &a, const SpecDyn *sd, const double *sca
    return 0.5 * ke / (ts * ts);
 }
 
-__device__ __forceinline__ void b_scalar(int bx, int nbx, const ScalArgs &a, const SpecDyn *__restrict__ sd,
-                                         const int *__restrict__ spec_rdof, const double *__restrict__ res,
-                                         double *__restrict__ scal, double *__restrict__ trace) {
-   if (threadIdx.x != 0 || bx != 0) return;
+__device__ __forceinline__ void b_scalar(int bx, int nbx, const ScalArgs &a, const SpecDyn *sd, const int *spec_rdof,
+                                         const double *res, const double *part, double *scal, double *trace) {
+   if (bx != 0) return;
+   if (a.ke_rows > 0) {
+      b_col_sum(0, 1, a.ke_rows, 4 * a.nspec, part, scal + S_KE);
+      __syncthreads();
+   }
+   if (threadIdx.x != 0) return;
    double &ts = scal[S_TS], &tsmom = scal[S_TSMOM];
    switch (a.op) {
       case OP_THERM_IN:
@@ -494,9 +534,9 @@ __device__ __forceinline__ void b_scalar(int bx, int nbx, const ScalArgs &a, con
       case OP_HMOM_VIR: update_hmom(a, a.step, ts, scal + S_H, res + 5, scal + S_HMOM); break;
    }
 }
-__global__ void k_scalar(ScalArgs a, const SpecDyn *__restrict__ sd, const int *__restrict__ spec_rdof,
-                         const double *__restrict__ res, double *__restrict__ scal, double *__restrict__ trace) {
-   b_scalar(blockIdx.x, gridDim.x, a, sd, spec_rdof, res, scal, trace);
+__global__ __launch_bounds__(256) void k_scalar(ScalArgs a, const SpecDyn *sd, const int *spec_rdof,
+                                                const double *res, const double *part, double *scal, double *trace) {
+   b_scalar(blockIdx.x, gridDim.x, a, sd, spec_rdof, res, part, scal, trace);
 }
 
 void matmul3(const double *a, const double *b, double *c) {
@@ -526,8 +566,8 @@ ScalArgs scal_args(mgpu_engine *e, int op) {
 }
 
 void scalar_op(mgpu_engine *e, const ScalArgs &a) {
-   glaunch<k_scalar, b_scalar, 1024>(e->rec, e->stream, 1, 64, 0, a, (const SpecDyn *)e->d_spec_dyn.p,
-                                     e->d_spec_rdof.p, e->d_out.p + OUT_RES, e->d_scal.p, e->d_trace.p);
+   glaunch<k_scalar, b_scalar, 256>(e->rec, e->stream, 1, 256, 0, a, (const SpecDyn *)e->d_spec_dyn.p,
+                                    e->d_spec_rdof.p, e->d_out.p + OUT_RES, e->d_red.p, e->d_scal.p, e->d_trace.p);
 }
 
 KeArgs ke_args(mgpu_engine *e) {
@@ -539,11 +579,13 @@ KeArgs ke_args(mgpu_engine *e) {
    return k;
 }
 
-void ke_sums(mgpu_engine *e) {
-   const int nb = (e->nmols + 255) / 256, nc = 4 * e->nspecies;
-   glaunch<k_ke_part, b_ke_part, 256>(e->rec, e->stream, nb, 256, 0, ke_args(e), e->d_mol_spec.p, e->d_mol_quat.p,
-                                      e->d_mom.p, e->d_amom.p, e->d_red.p);
-   glaunch<k_col_sum, b_col_sum, 256>(e->rec, e->stream, 1, 256, 0, nb, nc, e->d_red.p, e->d_scal.p + S_KE);
+// The kinetic sums, then the scalar update that needs them (which adds the
+// partials itself: one launch for two).
+void ke_scalar(mgpu_engine *e, ScalArgs a) {
+   a.ke_rows = (e->nmols + 255) / 256;
+   glaunch<k_ke_part, b_ke_part, 256>(e->rec, e->stream, a.ke_rows, 256, 0, ke_args(e), e->d_mol_spec.p,
+                                      e->d_mol_quat.p, e->d_mom.p, e->d_amom.p, e->d_red.p);
+   scalar_op(e, a);
 }
 
 void dyad_sums(mgpu_engine *e) {
@@ -553,9 +595,8 @@ void dyad_sums(mgpu_engine *e) {
    glaunch<k_col_sum, b_col_sum, 256>(e->rec, e->stream, 1, 256, 0, nb, nc, e->d_red.p, e->d_scal.p + S_DY);
 }
 
-// One leapf_all_coords half step, with the thermostat's rotational terms
-// between the rotation sub-steps when the thermostat is on.
-void coords_half(mgpu_engine *e) {
+// Arguments of a leapf_all_coords half step in one launch.
+CoordArgs coord_args(mgpu_engine *e) {
    CoordArgs c{};
    c.nmols = e->nmols;
    c.step = 0.5 * e->dyn_step;
@@ -566,6 +607,19 @@ void coords_half(mgpu_engine *e) {
    host_invert(G, c.Gi);
    c.variant_a = e->dyn_nosym;
    c.saxis = e->dyn_saxis;
+   c.do_com = 1;
+   c.ph_hi = e->nmols_r ? (e->dyn_nosym ? 5 : 3) : 0;
+   c.normalise = 1;
+   return c;
+}
+
+// The thermostat's rotational terms come between the rotation sub-steps.
+bool split_coords(const mgpu_engine *e) { return e->dyn_const_temp && e->nmols_r > 0; }
+
+// One leapf_all_coords half step, with the thermostat's rotational terms
+// between the rotation sub-steps when the thermostat is on.
+void coords_half(mgpu_engine *e) {
+   CoordArgs c = coord_args(e);
    const int nb = (e->nmols + 255) / 256;
    const int nph = e->dyn_nosym ? 5 : 3;
    auto launch = [&](int com, int lo, int hi) {
@@ -577,50 +631,69 @@ void coords_half(mgpu_engine *e) {
                                         (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p, e->d_mom.p, e->d_cm.p,
                                         e->d_quat.p, e->d_amom.p, e->d_iflags.p);
    };
-   if (!e->dyn_const_temp || e->nmols_r == 0) {
-      launch(1, 0, e->nmols_r ? nph : 0);
+   if (!split_coords(e)) {
+      launch(1, 0, c.ph_hi);
       return;
    }
    if (!e->dyn_nosym) {
       launch(1, 0, 1);
-      ke_sums(e);
       ScalArgs a = scal_args(e, OP_TSMOM_ROT);
       a.step = c.step;
-      scalar_op(e, a);
+      ke_scalar(e, a);
       launch(0, 1, 2);
-      ke_sums(e);
-      scalar_op(e, a);
+      ke_scalar(e, a);
       launch(0, 2, 3);
    } else {
       // leapf_quat_a: sums after sub-steps 0, 1 and 3
       launch(1, 0, 1);
-      ke_sums(e);
       ScalArgs a = scal_args(e, OP_TSMOM_AXES);
       a.step = c.step;
       a.naxes = 2; a.axes[0] = 0; a.axes[1] = 1; a.w[0] = 0.25; a.w[1] = 0.25;
-      scalar_op(e, a);
+      ke_scalar(e, a);
       launch(0, 1, 2);
-      ke_sums(e);
       a.naxes = 1; a.axes[0] = 2; a.w[0] = 0.5;
-      scalar_op(e, a);
+      ke_scalar(e, a);
       launch(0, 2, 4);
-      ke_sums(e);
       a.naxes = 2; a.axes[0] = 1; a.axes[1] = 0; a.w[0] = 0.25; a.w[1] = 0.25;
-      scalar_op(e, a);
+      ke_scalar(e, a);
       launch(0, 4, 5);
    }
 }
 
-void momenta_half(mgpu_engine *e, bool zero_fw) {
+MomArgs mom_args(mgpu_engine *e, bool zero_fw) {
    MomArgs m{};
    m.nmols = e->nmols;
    m.step = 0.5 * e->dyn_step;
    for (int i = 0; i < 3; i++)
       for (int j = 0; j < 3; j++) m.hT[3 * i + j] = e->h[3 * j + i];
    m.zero_fw = zero_fw;
-   glaunch<k_momenta, b_momenta, 1024>(e->rec, e->stream, (e->nmols + 255) / 256, 256, 0, m, e->d_mol_spec.p,
-                                       e->d_mol_quat.p, (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p, e->d_mforce.p,
-                                       e->d_mtorque.p, e->d_mom.p, e->d_amom.p);
+   return m;
+}
+
+// The first momentum half step, the kinetic sums and the step's record.
+void momenta_record(mgpu_engine *e) {
+   ScalArgs a = scal_args(e, OP_RECORD);
+   a.ke_rows = (e->nmols + 255) / 256;
+   glaunch<k_mom_ke, b_mom_ke, 256>(e->rec, e->stream, a.ke_rows, 256, 0, mom_args(e, false), ke_args(e),
+                                    e->d_mol_spec.p, e->d_mol_quat.p, (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p,
+                                    e->d_mforce.p, e->d_mtorque.p, e->d_mom.p, e->d_amom.p, e->d_red.p);
+   scalar_op(e, a);
+}
+
+// The second momentum half step.
+void momenta_half(mgpu_engine *e) {
+   glaunch<k_momenta, b_momenta, 256>(e->rec, e->stream, (e->nmols + 255) / 256, 256, 0, mom_args(e, true),
+                                      e->d_mol_spec.p, e->d_mol_quat.p, (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p,
+                                      e->d_mforce.p, e->d_mtorque.p, e->d_mom.p, e->d_amom.p);
+}
+
+// The second momentum half step and the coordinate half step after it, with
+// no thermostat between them.
+void momenta_coords(mgpu_engine *e) {
+   glaunch<k_mom_coords, b_mom_coords, 256>(
+       e->rec, e->stream, (e->nmols + 255) / 256, 256, 0, mom_args(e, true), coord_args(e), e->d_mol_spec.p,
+       e->d_mol_quat.p, (const SpecDyn *)e->d_spec_dyn.p, e->d_scal.p, e->d_mforce.p, e->d_mtorque.p, e->d_mom.p,
+       e->d_cm.p, e->d_quat.p, e->d_amom.p, e->d_iflags.p);
 }
 
 }  // namespace
@@ -743,24 +816,22 @@ void mgpu::md_reset_record(mgpu_engine *e, int cap, bool init_h0) {
 // no host synchronisation.
 void mgpu::md_step_launch(mgpu_engine *e) {
    const bool therm = e->dyn_const_temp;
-   if (therm) scalar_op(e, scal_args(e, OP_THERM_IN));
    if (therm) {
-      ke_sums(e);
-      scalar_op(e, scal_args(e, OP_TSMOM_TRANS));
+      scalar_op(e, scal_args(e, OP_THERM_IN));
+      ke_scalar(e, scal_args(e, OP_TSMOM_TRANS));
    }
    coords_half(e);
    eval_forces_device(e, false);
-   momenta_half(e, false);
-   ke_sums(e);
-   scalar_op(e, scal_args(e, OP_RECORD));
-   momenta_half(e, true);
-   if (therm) scalar_op(e, scal_args(e, OP_TSMOM_PE));
-   if (therm) {
-      ke_sums(e);
-      scalar_op(e, scal_args(e, OP_TSMOM_TRANS));
+   momenta_record(e);
+   if (!therm) {
+      momenta_coords(e);
+      return;
    }
+   momenta_half(e);
+   scalar_op(e, scal_args(e, OP_TSMOM_PE));
+   ke_scalar(e, scal_args(e, OP_TSMOM_TRANS));
    coords_half(e);
-   if (therm) scalar_op(e, scal_args(e, OP_THERM_OUT));
+   scalar_op(e, scal_args(e, OP_THERM_OUT));
 }
 
 // do_step with the barostat (const_pressure branches of src/accel.c:686-779).
@@ -774,22 +845,18 @@ void mgpu::md_step_pressure(mgpu_engine *e) {
    md_fetch_cell(e, h, nullptr);
    set_geometry(e, h);
    if (therm) {
-      ke_sums(e);
-      scalar_op(e, scal_args(e, OP_TSMOM_TRANS));
+      ke_scalar(e, scal_args(e, OP_TSMOM_TRANS));
    }
    dyad_sums(e);
    scalar_op(e, scal_args(e, OP_HMOM_KIN));
    coords_half(e);
    eval_forces_device(e, false);
-   momenta_half(e, false);
-   ke_sums(e);
-   scalar_op(e, scal_args(e, OP_RECORD));
-   momenta_half(e, true);
+   momenta_record(e);
+   momenta_half(e);
    if (therm) scalar_op(e, scal_args(e, OP_TSMOM_PE));
    scalar_op(e, scal_args(e, OP_HMOM_VIR));
    if (therm) {
-      ke_sums(e);
-      scalar_op(e, scal_args(e, OP_TSMOM_TRANS));
+      ke_scalar(e, scal_args(e, OP_TSMOM_TRANS));
    }
    dyad_sums(e);
    scalar_op(e, scal_args(e, OP_HMOM_KIN));
