@@ -415,7 +415,9 @@ def main():
     evals = 1.0 / t
     res.update(value=evals, unit="force-evals/s", ms_per_step=1e3 * t,
                ns_per_day=evals * DT_FS * 86400 / 1e6,
-               dtype="f32 pairs + f16x2 MFMA Ewald + f64 reductions" if mixed else "f64",
+               dtype=("f64" if not mixed else
+                      "f32 pairs + f16x2 MFMA Ewald + f64 reductions" if "ewald_mfma_force" in mixed["prof"] else
+                      "f32 pairs + f32 gridded Ewald with f64 transforms + f64 reductions"),
                config=dict(workload=f"aqueous MgCl2: 32768 rigid 4-site water + 600 Mg2+ + 1200 Cl- "
                                     f"({ns} sites)", sites=ns, k_vectors=nk, cutoff_A=10.0,
                            alpha_per_A=0.30, k_cutoff_per_A=round(s.control.k_cutoff, 4),
