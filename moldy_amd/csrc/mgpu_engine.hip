@@ -713,10 +713,11 @@ void mgpu::eval_forces_device(mgpu_engine *e, bool clear_flags) {
    // flag is cleared however this function is left
    struct DeferRecip {
       mgpu_engine *e;
-      ~DeferRecip() { e->defer_recip = false; }
+      ~DeferRecip() { e->defer_recip = e->defer_real = false; }
    } defer_guard{e};
    e->defer_recip = !e->surface_dipole && e->precision == MGPU_MIXED;
-   e->recip_part = nullptr;
+   e->defer_real = !e->surface_dipole;
+   e->recip_part = e->real_part = nullptr;
    if (e->overlap && e->alpha > 1e-7) {
       HIPCHK(hipEventRecord(e->ev_fork, e->stream));
       HIPCHK(hipStreamWaitEvent(e->side, e->ev_fork, 0));
@@ -739,7 +740,7 @@ void mgpu::eval_forces_device(mgpu_engine *e, bool clear_flags) {
       real_pass_device(e, false, true);
       if (e->alpha > 1e-7) recip_pass_device(e);
    }
-   e->defer_recip = false;
+   e->defer_recip = e->defer_real = false;
    run_glue(e);
 }
 

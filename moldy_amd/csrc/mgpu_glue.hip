@@ -470,20 +470,28 @@ __global__ __launch_bounds__(256) void k_glue_parts(GlueArgs g, const int *__res
 // q, q + 48, ... in order, then those 48 sums in order; thread 0 assembles.
 // With rpart set, also the reciprocal pass's 8 sums (OUT_RECIP) from its
 // rrows rows of per-block partials: 128 threads a column add every 128th
-// row in order, then those 128 sums in order (before the assembly reads them).
+// row in order, then those 128 sums in order (before the assembly reads them);
+// with qpart set, the real-space pass's (OUT_REAL) likewise.
 __device__ __forceinline__ void b_glue_sum(int bx, int nbx, const AsmArgs &a, int nb, int nmb,
                                            const double *__restrict__ part_s, const double *__restrict__ part_m,
-                                           const double *__restrict__ rpart, int rrows, double *__restrict__ out) {
+                                           const double *__restrict__ rpart, int rrows,
+                                           const double *__restrict__ qpart, int qrows, double *__restrict__ out) {
    constexpr int NC = GLUE_S + GLUE_M, NT = 48, RT = 128;
    __shared__ double sp[NC][NT];
    __shared__ double col[NC];
-   __shared__ double rp[8][RT];
+   __shared__ double rp[8][RT], qp[8][RT];
    const int t = threadIdx.x;
    if (rpart) {
       const int c = t / RT, q = t - c * RT;
       double acc = 0.0;
       for (int r = q; r < rrows; r += RT) acc += rpart[(size_t)r * 8 + c];
       rp[c][q] = acc;
+   }
+   if (qpart) {
+      const int c = t / RT, q = t - c * RT;
+      double acc = 0.0;
+      for (int r = q; r < qrows; r += RT) acc += qpart[(size_t)r * 8 + c];
+      qp[c][q] = acc;
    }
    if (t < NC * NT) {
       const int c = t / NT, q = t - c * NT;
@@ -503,6 +511,10 @@ __device__ __forceinline__ void b_glue_sum(int bx, int nbx, const AsmArgs &a, in
       double acc = 0.0;
       for (int q = 0; q < RT; q++) acc += rp[t - 32][q];
       out[OUT_RECIP + (t - 32)] = acc;
+   } else if (qpart && t >= 64 && t < 72) {
+      double acc = 0.0;
+      for (int q = 0; q < RT; q++) acc += qp[t - 64][q];
+      out[OUT_REAL + (t - 64)] = acc;
    }
    __syncthreads();
    if (t == 0) {
@@ -514,8 +526,9 @@ __device__ __forceinline__ void b_glue_sum(int bx, int nbx, const AsmArgs &a, in
 }
 __global__ __launch_bounds__(1024) void k_glue_sum(AsmArgs a, int nb, int nmb, const double *__restrict__ part_s,
                                                    const double *__restrict__ part_m, const double *__restrict__ rpart,
-                                                   int rrows, double *__restrict__ out) {
-   b_glue_sum(blockIdx.x, gridDim.x, a, nb, nmb, part_s, part_m, rpart, rrows, out);
+                                                   int rrows, const double *__restrict__ qpart, int qrows,
+                                                   double *__restrict__ out) {
+   b_glue_sum(blockIdx.x, gridDim.x, a, nb, nmb, part_s, part_m, rpart, rrows, qpart, qrows, out);
 }
 
 }  // namespace
@@ -576,8 +589,8 @@ void mgpu::run_glue(mgpu_engine *e) {
                                                e->d_chg_site.p, e->d_force_site.p, e->d_site.p, e->d_mforce.p,
                                                e->d_mtorque.p, part_s, part_m);
       glaunch<k_glue_sum, b_glue_sum, 1024>(e->rec, e->stream, 1, 1024, 0, aa, nb, nmb1, part_s, part_m,
-                                            e->recip_part, e->recip_rows, out);
-      e->recip_part = nullptr;
+                                            e->recip_part, e->recip_rows, e->real_part, e->real_rows, out);
+      e->recip_part = e->real_part = nullptr;
       return;
    }
    // second make_sites: MOLPBC for molecules, SITEPBC for frameworks (accel.c:536-541)

@@ -247,6 +247,10 @@ struct mgpu_engine {
    bool defer_recip = false;
    const double *recip_part = nullptr;
    int recip_rows = 0;
+   // the same for a real-space pass of few rows
+   bool defer_real = false;
+   const double *real_part = nullptr;
+   int real_rows = 0;
 
    // ---- molecular dynamics (device-resident state of the integrator) ----
    bool have_dyn = false;

@@ -981,5 +981,12 @@ void mgpu::run_realspace(mgpu_engine *e) {
       }
    }
    e->d_out.reserve(OUT_SIZE);
-   reduce_cols(e, e->d_cell_part.p, nwaves, 8, e->d_out.p + OUT_REAL);
+   if (e->defer_real && nwaves <= 2048) {
+      // few rows: the glue adds them beside its own (16 loads a thread at the
+      // most), where a column sum is a launch of 7.5 us (864 argon atoms)
+      e->real_part = e->d_cell_part.p;
+      e->real_rows = nwaves;
+   } else {
+      reduce_cols(e, e->d_cell_part.p, nwaves, 8, e->d_out.p + OUT_REAL);
+   }
 }
