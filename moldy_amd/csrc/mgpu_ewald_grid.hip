@@ -118,8 +118,10 @@ __device__ __forceinline__ void b_g_bin(int bx, int nbx, const GBinArgs &a) {
          hi = t;
       }
       hi -= rint(hi);
-      if (!(fabs(hi) <= 0.5)) hi = lo = 0.0;   // not a number
-      const double n = a.n[d], hw = 0.5 * a.w, c = ceil(__builtin_fma(n, hi, -hw));
+      // a coordinate that is not finite is put into the origin's brick, and its
+      // argument stays NaN: its weights, and with them all sums, are NaN then,
+      // as the direct sum's are
+      const double n = a.n[d], hw = 0.5 * a.w, c = ceil(__builtin_fma(n, fabs(hi) <= 0.5 ? hi : 0.0, -hw));
       an[d] = (int)c;
       if (an[d] < 0) an[d] += a.n[d];
       a.sx[(size_t)d * a.nsp + i] = 2.0 * (__builtin_fma(-n, hi, c + hw) - n * lo) - 1.0;

@@ -34,6 +34,12 @@ def _system(name):
     return system.silica(ncell=10, seed=14, cutoff=10.0)
 
 
+def _past_rule(prec):
+    """Just past the size rule of each precision."""
+    from moldy_amd import engine as E, system
+    return system.water_box(3600 if prec == E.FP64 else 5000, seed=11)
+
+
 def _check(s, xyz, prec, tol_f, tol_e):
     from moldy_amd import engine as E
     from oracle.oracle import Oracle
@@ -93,3 +99,34 @@ def test_placement(case):
 def test_noalloc_takes_the_same_path():
     import test_zz_no_alloc as T
     T._compare(_system("water"), 6)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("prec", [0, 1])
+def test_coordinate_not_finite(bad, prec):
+    """One site without a place makes every sum NaN, as in the direct sum (its
+    phase enters every S(k)); the engine's next call is not touched by it."""
+    from moldy_amd import engine as E
+    from oracle.oracle import Oracle
+    import test_zz_no_alloc as T
+    s = _past_rule(prec)
+    xyz = Oracle(s).make_sites()
+    e = E.ForceEngine(s, precision=prec)
+    zero = np.zeros((3, s.nsites))
+    calls = ["mgpu_ewald"] + (["mgpu_ewald_noalloc"] if prec == E.FP64 else [])
+    good = {}
+    for name in calls:
+        rc, f, pe, st, _ = T._call(e, name, s, xyz, zero)
+        assert rc == 0 and np.all(np.isfinite(f)) and np.isfinite(pe)
+        good[name] = (f, pe, st)
+    for axis in range(3):
+        x = xyz.copy()
+        x[axis, 17 + axis] = bad
+        for name in calls:
+            rc, f, pe, st, _ = T._call(e, name, s, x, zero)
+            assert rc == 0
+            assert np.all(np.isnan(f)) and np.isnan(pe) and np.all(np.isnan(st[[0, 4, 8]])), (name, axis)
+    for name in calls:
+        rc, f, pe, st, _ = T._call(e, name, s, xyz, zero)
+        assert np.array_equal(f, good[name][0]) and pe == good[name][1] and np.array_equal(st, good[name][2])
+    e.close()
