@@ -15,10 +15,14 @@
 //   window   phi(z) = exp(beta (sqrt(1 - z^2) - 1)), |z| <= 1, z = 2 d / w for a
 //            grid distance d (the "exponential of semicircle" window of
 //            Barnett, Magland and af Klinteberg, SIAM J. Sci. Comput. 41, C479,
-//            2019).  beta = 2.5 w (FP64) and 2.6 w (FP32): past their 2.3 w,
+//            2019).  beta = 2.6 w (FP64) and 2.7 w (FP32): past their 2.3 w,
 //            because the Ewald weight exp(-k^2/4 alpha^2) damps the k next to
 //            the cutoff, whose aliases a larger beta raises, while the
-//            derivative of the window at its edge falls.  It is evaluated as one polynomial per grid offset.
+//            window's jump at its edge falls.  Its own error in the forces
+//            of 4,054 salt water sites (all else in long double): 1.5e-15 at
+//            2.5 w, 4e-16 at 2.6 w, 5e-16 at 2.65 w; for FP32 2.9e-7 at 2.6 w,
+//            1.4e-7 at 2.7 w, 1.1e-7 at 2.75 w (1.2e-7 and rising in silica).
+//            It is evaluated as one polynomial per grid offset.
 //   spread   G(x,y,z) = sum_i q_i phi phi phi
 //   forward  T(h,k,l) = sum_xyz G e^{+2 pi i (hx/nx + ky/ny + lz/nz)}, l >= 0, as
 //            dense transforms of one axis at a time on the matrix cores: only the
@@ -52,11 +56,11 @@ constexpr int GB = 8;               // brick edge in grid points
 template <class R> struct Win;
 template <> struct Win<double> {
    static constexpr int W = 16, DEG = 15;
-   static constexpr double BETA = 2.5 * W;
+   static constexpr double BETA = 2.6 * W;
 };
 template <> struct Win<float> {
    static constexpr int W = 8, DEG = 10;
-   static constexpr double BETA = 2.6 * W;
+   static constexpr double BETA = 2.7 * W;
 };
 // A site's spread weights: three rows of W + 2, a zero at either end for every
 // grid point outside the window.
@@ -849,7 +853,7 @@ GridGeom mgpu::grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const do
    for (int d = 0; d < 3; d++) {
       // grid points per shortest wave along this cell vector (kc |h_d| / 2 pi
       // waves): the aliases of the modes next to the cutoff are down by
-      // phi^(n - m) / phi^(m) = 3e-14 at 4.6 (FP64), 2e-5 at 4 (FP32), before
+      // phi^(n - m) / phi^(m) = 1.4e-11 at 4.6 (FP64), 1.1e-4 at 4 (FP32), before
       // the weight's own 1e-6
       const double wv = kc / (2 * PI_D) * sqrt(h[d] * h[d] + h[3 + d] * h[3 + d] + h[6 + d] * h[6 + d]);
       g.n[d] = (int)std::min(1e6, std::max(3.0 * GB, ceil((fp64 ? 4.6 : 4.0) * wv / GB) * GB));
