@@ -20,6 +20,8 @@
 #include "mgpu_internal.h"
 #include "mgpu_pair.h"
 
+#include <type_traits>
+
 using namespace mgpu;
 
 namespace {
@@ -267,12 +269,18 @@ __device__ __forceinline__ int dpp_scan(int x) {
    return x;
 }
 
+// S64 (FP32 pairs): a lane adds every pair's force, energy and virial in FP64, as
+// the walk adds each cell's, instead of keeping FP32 sums over the 11 or so pairs of a
+// site that it meets.  Forces of 216 to 912 waters against FP64: 1.6 to 2.3% closer,
+// as the walk's to 0.1%; the kernel alone 2,048 sites 12 us either way, 132,872 sites
+// 222 and 232 us.
 // MC: groups of 64 columns (2 holds the shell of a near-cubic cell at the
 // reference's subcell, about 110 columns; 4 the most, 256).
-template <class R, int PT, bool COUL, int MC, class A = const RSArgs &>
+template <class R, int PT, bool COUL, int MC, bool S64, class A = const RSArgs &>
 __device__ __forceinline__ void b_realspace_bal(int bx, int nbx, A a) {
    constexpr bool F4 = sizeof(R) == 4;
    constexpr int ND = RSB_ND<R>;
+   using S = typename std::conditional<S64, double, R>::type;
    extern __shared__ __attribute__((aligned(16))) unsigned char rsb_lds[];
    const int npp = a.max_id * a.max_id * MGPU_NPOTP, maxp = 2 * a.ncol;
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -386,7 +394,8 @@ __device__ __forceinline__ void b_realspace_bal(int bx, int nbx, A a) {
       }
       cself = __builtin_amdgcn_readlane(cself, a.own_col & 63);
 
-      R fx = 0, fy = 0, fz = 0, ep = 0, w00 = 0, w01 = 0, w02 = 0, w11 = 0, w12 = 0, w22 = 0;
+      S fx = 0, fy = 0, fz = 0;
+      R ep = 0, w00 = 0, w01 = 0, w02 = 0, w11 = 0, w12 = 0, w22 = 0;
       int nst = -1;   // piece starts before the batch, less one
       // windows of candidates: a bit per piece start, then the window's batches of 64
       for (int wbase = 0; wbase < total; wbase += 64 * a.bit_words) {   // uniform
@@ -462,19 +471,27 @@ __device__ __forceinline__ void b_realspace_bal(int bx, int nbx, A a) {
                f = 0;
             }
             const R gx = f * rx, gy = f * ry, gz = f * rz;
-            fx -= gx;
-            fy -= gy;
-            fz -= gz;
-            ep += u;
-            w00 += gx * rx; w01 += gx * ry; w02 += gx * rz;
-            w11 += gy * ry; w12 += gy * rz; w22 += gz * rz;
+            if constexpr (S64) {
+               fx -= (double)gx; fy -= (double)gy; fz -= (double)gz;
+               v[0] += (double)u;
+               v[1] += (double)(gx * rx); v[2] += (double)(gx * ry); v[3] += (double)(gx * rz);
+               v[4] += (double)(gy * ry); v[5] += (double)(gy * rz); v[6] += (double)(gz * rz);
+            } else {
+               // from f, so that the product is not rounded by itself
+               fx -= f * rx; fy -= f * ry; fz -= f * rz;
+               ep += u;
+               w00 += gx * rx; w01 += gx * ry; w02 += gx * rz;
+               w11 += gy * ry; w12 += gy * rz; w22 += gz * rz;
+            }
          }
       }
       double gx = (double)fx, gy = (double)fy, gz = (double)fz;
       wave_sum3(gx, gy, gz, lane);
-      v[0] += (double)ep;
-      v[1] += (double)w00; v[2] += (double)w01; v[3] += (double)w02;
-      v[4] += (double)w11; v[5] += (double)w12; v[6] += (double)w22;
+      if constexpr (!S64) {
+         v[0] += (double)ep;
+         v[1] += (double)w00; v[2] += (double)w01; v[3] += (double)w02;
+         v[4] += (double)w11; v[5] += (double)w12; v[6] += (double)w22;
+      }
       if (lane < 3) a.force[(size_t)lane * a.nsp + a.corig[p]] += lane == 0 ? gx : lane == 1 ? gy : gz;
    }
    double *pp = a.part + 8 * (size_t)row;
@@ -488,9 +505,9 @@ __device__ __forceinline__ void b_realspace_bal(int bx, int nbx, A a) {
 // Waves a SIMD the registers are held to (the compiler would take 133 in FP64 and
 // 87 in FP32 for two groups of columns, three and five waves).
 template <class R, int MC> constexpr int RSB_WPE = MC == 2 ? (sizeof(R) == 8 ? 4 : 6) : (sizeof(R) == 8 ? 3 : 4);
-template <class R, int PT, bool COUL, int MC>
+template <class R, int PT, bool COUL, int MC, bool S64>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RSB_WPE<R, MC>))) void k_realspace_bal(RSArgs a) {
-   b_realspace_bal<R, PT, COUL, MC, RSArgs>(blockIdx.x, gridDim.x, a);
+   b_realspace_bal<R, PT, COUL, MC, S64, RSArgs>(blockIdx.x, gridDim.x, a);
 }
 
 // Tiled Newton-3 variant: every pair once.  The full shell is symmetric,
@@ -861,8 +878,22 @@ __global__ __launch_bounds__(256) void k_rs_fold(const R *__restrict__ P, int nr
    b_rs_fold<R>(blockIdx.x, gridDim.x, P, nrows, nsites, nsp, corig, force);
 }
 
+template <class R, int PT, bool COUL, int MC>
+void launch_bal(std::vector<LaunchRec> *rec, bool s64, unsigned g, unsigned b, hipStream_t s, size_t shm,
+                const RSArgs &a) {
+   auto run = [&](auto S) {
+      constexpr bool S64 = decltype(S)::value;
+      glaunch<k_realspace_bal<R, PT, COUL, MC, S64>, b_realspace_bal<R, PT, COUL, MC, S64>, 256, RSB_WPE<R, MC>>(
+          rec, s, g, b, shm, a);
+   };
+   if constexpr (sizeof(R) == 4) {
+      if (s64) return run(std::true_type{});
+   }
+   run(std::false_type{});
+}
+
 template <class R, bool COUL>
-void launch_pt(std::vector<LaunchRec> *rec, int pt, int kind, unsigned g, unsigned b, hipStream_t s,
+void launch_pt(std::vector<LaunchRec> *rec, int pt, int kind, bool s64, unsigned g, unsigned b, hipStream_t s,
                const RSArgs &a) {
    const int npp = a.max_id * a.max_id * MGPU_NPOTP;
    const size_t shm = kind == 1   ? rsb_lds_bytes<R>(2 * a.ncol, npp)
@@ -872,9 +903,9 @@ void launch_pt(std::vector<LaunchRec> *rec, int pt, int kind, unsigned g, unsign
    case n:                                                                                             \
       if (kind == 1) {                                                                                 \
          if (a.ncol <= 128)                                                                            \
-            glaunch<k_realspace_bal<R, n, COUL, 2>, b_realspace_bal<R, n, COUL, 2>, 256, RSB_WPE<R, 2>>(rec, s, g, b, shm, a); \
+            launch_bal<R, n, COUL, 2>(rec, s64, g, b, s, shm, a);                                      \
          else                                                                                          \
-            glaunch<k_realspace_bal<R, n, COUL, 4>, b_realspace_bal<R, n, COUL, 4>, 256, RSB_WPE<R, 4>>(rec, s, g, b, shm, a); \
+            launch_bal<R, n, COUL, 4>(rec, s64, g, b, s, shm, a);                                      \
       } else if (kind == 2)                                                                            \
          glaunch<k_realspace_n3<R, n, COUL>, b_realspace_n3<R, n, COUL>, 256>(rec, s, g, b, shm, a);   \
       else                                                                                             \
@@ -959,14 +990,17 @@ void mgpu::run_realspace(mgpu_engine *e) {
    a.tooclose = e->d_iflags.p + 1;
    const unsigned g = nblk, b = 256;
    bool coul = e->alpha > 0.0;
+   // FP64 sums of the FP32 pairs where the walk, which has them, was the choice
+   // by speed before the balanced kernel was: they cost nothing there
+   const bool s64 = (long)e->nsites < 16L * e->ncu;
    {
       ProfScope ps(e, "realspace");
       if (e->precision == MGPU_FP64) {
-         if (coul) launch_pt<double, true>(e->rec, e->ptype, kind, g, b, e->stream, a);
-         else launch_pt<double, false>(e->rec, e->ptype, kind, g, b, e->stream, a);
+         if (coul) launch_pt<double, true>(e->rec, e->ptype, kind, s64, g, b, e->stream, a);
+         else launch_pt<double, false>(e->rec, e->ptype, kind, s64, g, b, e->stream, a);
       } else {
-         if (coul) launch_pt<float, true>(e->rec, e->ptype, kind, g, b, e->stream, a);
-         else launch_pt<float, false>(e->rec, e->ptype, kind, g, b, e->stream, a);
+         if (coul) launch_pt<float, true>(e->rec, e->ptype, kind, s64, g, b, e->stream, a);
+         else launch_pt<float, false>(e->rec, e->ptype, kind, s64, g, b, e->stream, a);
       }
       if (tile) {
          const int fb = (e->nsites + 255) / 256;

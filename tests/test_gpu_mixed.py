@@ -79,3 +79,27 @@ def test_mixed_one_group_backprojection():
     assert rel_err(rmx["stress"], r64["stress"]) < TOL_S
     e64.close()
     emx.close()
+
+
+@pytest.mark.parametrize("name", ["water216", "water512", "water729", "salt900"])
+def test_small_systems_keep_fp64_sums_of_pairs(name):
+    """Below 16 sites a CU the balanced kernel sums FP32 pairs in FP64, as the
+    walk does: the same error against FP64 to 0.5% (FP32 sums over a lane's pairs
+    of a site were 1.6 to 2.3% off; all runs are deterministic).  The energy is a
+    sum of 1e5 pairs whose rounding errors cancel at random: not compared."""
+    from moldy_amd import engine as E, system
+    s = (system.salt_water(nwater=900, nmg=16, ncl=32, seed=7) if name == "salt900"
+         else system.water_box(int(name[5:]), seed=5))
+    e = E.ForceEngine(s, precision=E.FP64)
+    xyz = e.eval_forces()["site_xyz"]
+    ref = e.force_calc(s.h, xyz)["force"]
+    e.close()
+    err = {}
+    for mode in (E.ForceEngine.RS_AUTO, E.ForceEngine.RS_WALK):
+        e = E.ForceEngine(s, precision=E.MIXED)
+        e.set_realspace_mode(mode)
+        err[mode] = rel_err(e.force_calc(s.h, xyz)["force"], ref)
+        assert e.realspace_balanced() == (mode == E.ForceEngine.RS_AUTO)
+        e.close()
+    print(name, {k: f"{v:.4e}" for k, v in err.items()})
+    assert err[E.ForceEngine.RS_AUTO] < 1.005 * err[E.ForceEngine.RS_WALK]
