@@ -321,9 +321,7 @@ __global__ __launch_bounds__(256) void k_adj_fold(int nw, int max_id, int npar, 
 }
 
 template <int PT, bool COUL> void launch_adj(unsigned g, size_t shm, hipStream_t s, const AdjArgs &a) {
-   if (shm > 64 * 1024)
-      HIPCHK(hipFuncSetAttribute((const void *)k_adj_real<PT, COUL>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)shm));
+   allow_lds((const void *)k_adj_real<PT, COUL>, shm);
    k_adj_real<PT, COUL><<<g, 64, shm, s>>>(a);
 }
 

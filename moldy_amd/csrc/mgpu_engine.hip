@@ -547,6 +547,11 @@ void pin_free(PinBuf &b) {
 }
 }  // namespace
 
+void mgpu::allow_lds(const void *kernel, size_t shm) {
+   if (shm > 64 * 1024)
+      HIPCHK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+}
+
 // A copy from pageable memory waits for itself, and every upload waited for the
 // stream: 24 replicas of 256 to 2,048 waters spent 1.6 ms a call in 240 such
 // copies.

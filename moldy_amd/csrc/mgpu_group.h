@@ -116,10 +116,19 @@ struct LaunchRec {
    std::vector<char> args;
 };
 
+// Lets kernel take shm bytes of dynamic LDS: past 64 KiB a launch needs the
+// limit raised first.
+void allow_lds(const void *kernel, size_t shm);
+
 template <auto Body, int LB, int WPE>
 void launch_group(const GroupTab &t, unsigned grid, unsigned block, size_t shm, hipStream_t s) {
-   if constexpr (WPE > 0) k_grouped_w<Body, LB, WPE><<<grid, block, shm, s>>>(t);
-   else k_grouped<Body, LB><<<grid, block, shm, s>>>(t);
+   if constexpr (WPE > 0) {
+      allow_lds((const void *)k_grouped_w<Body, LB, WPE>, shm);
+      k_grouped_w<Body, LB, WPE><<<grid, block, shm, s>>>(t);
+   } else {
+      allow_lds((const void *)k_grouped<Body, LB>, shm);
+      k_grouped<Body, LB><<<grid, block, shm, s>>>(t);
+   }
 }
 
 // Launch K directly, or append the launch to rec.  LB (and WPE) must be the
@@ -128,6 +137,7 @@ void launch_group(const GroupTab &t, unsigned grid, unsigned block, size_t shm, 
 template <auto K, auto Body, int LB, int WPE = 0, class... A>
 void glaunch(std::vector<LaunchRec> *rec, hipStream_t s, unsigned grid, unsigned block, size_t shm, A &&...args) {
    if (!rec) {
+      allow_lds((const void *)K, shm);
       K<<<grid, block, shm, s>>>(std::forward<A>(args)...);
       return;
    }
