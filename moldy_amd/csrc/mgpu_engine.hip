@@ -1088,6 +1088,7 @@ int mgpu_ewald(mgpu_engine *e, const double h[9], const double *site, int ld, co
 int mgpu_upload_state(mgpu_engine *e, const double h[9], const double *cm, const double *quat) {
    return guarded(e, [&] {
       if (!e->have_system) return fail(e, MGPU_E_STATE, "mgpu_set_system not called");
+      if (!h || !cm || (e->nmols_r && !quat)) return fail(e, MGPU_E_ARG, "bad buffers");
       HIPCHK(hipSetDevice(e->device));
       set_geometry(e, h);
       const double *src[2] = {cm, quat};

@@ -46,6 +46,33 @@ def test_replayed_first_step_is_bitwise_eager(prec, nvt):
     e.close()
 
 
+def test_upload_without_a_buffer_is_an_error():
+    """Missing arrays are refused with a status (the copy into pinned memory
+    would read them), and the engine goes on as it was."""
+    import ctypes as C
+    from moldy_amd import engine as E, system
+    s = system.water_box(64, seed=21, cutoff=5.5, alpha=0.40)
+    e = E.ForceEngine(s)
+    want = e.eval_forces()
+    L, dp = E.lib(), C.POINTER(C.c_double)
+    h, cm, q = (np.ascontiguousarray(x, np.float64) for x in (s.h, s.c_of_m, s.quat))
+    p = [x.ctypes.data_as(dp) for x in (h, cm, q)]
+    for missing in range(3):
+        args = [None if k == missing else p[k] for k in range(3)]
+        assert L.mgpu_upload_state(e.h_, *args) == 1      # MGPU_E_ARG
+        assert b"bad buffers" in L.mgpu_last_error(e.h_)
+    pe, dip, st = e.eval_forces_device()
+    assert np.array_equal(pe, want["pe"]) and np.array_equal(st, want["stress"])
+    # atoms have no quaternions to give
+    a = system.argon_fcc(4, cutoff=8.5)
+    ea = E.ForceEngine(a)
+    h, cm = np.ascontiguousarray(a.h), np.ascontiguousarray(a.c_of_m)
+    assert L.mgpu_upload_state(ea.h_, h.ctypes.data_as(dp), cm.ctypes.data_as(dp), None) == 0
+    ea.eval_forces_device()
+    e.close()
+    ea.close()
+
+
 def test_replay_after_another_precision():
     """A captured mixed step, an FP64 evaluation (other tables of the gridded
     reciprocal sum), then the mixed run again: the capture is not reused with
