@@ -862,8 +862,12 @@ GridGeom mgpu::grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const do
    for (int i = 0; i < 9; i++) g.hinv[i] = hinv[i];
    g.vol = vol; g.alpha = alpha;
    g.w = fp64 ? Win<double>::W : Win<float>::W;
+   // a brick's bucket holds four times the mean count and what a dense liquid's
+   // or solid's 0.2 sites an A^3 put there (a droplet's bricks are full while the mean
+   // is low), up to 448 (LDS of the weights kernel)
    const long nbr = (long)g.nb[0] * g.nb[1] * g.nb[2];
-   g.cap = up((int)std::min(448L, std::max(64L, 4 * (ns / nbr + 1))), 64);
+   const double fill = std::max(4.0 * (ns / nbr + 1), std::min(0.2 * vol / nbr, (double)ns));
+   g.cap = up((int)std::min(448.0, std::max(64.0, fill)), 64);
    return g;
 }
 

@@ -195,3 +195,54 @@ def test_coordinate_not_finite(bad, prec):
         rc, f, pe, st, _ = T._call(e, name, s, xyz, zero)
         assert np.array_equal(f, good[name][0]) and pe == good[name][1] and np.array_equal(st, good[name][2])
     e.close()
+
+
+def _took_grid(e):
+    """Whether the last evaluation or ewald call with profiling on took the grid."""
+    return e.profile_get("ewald_grid_spread")[1] > 0
+
+
+def _route(s, prec):
+    from moldy_amd import engine as E
+    e = E.ForceEngine(s, precision=prec)
+    e.profile(True)
+    e.upload_state()
+    e.eval_forces_device()
+    grid = _took_grid(e)
+    e.close()
+    return grid
+
+
+def _droplet(n, widen, alpha):
+    """Liquid water in the middle of a box widen times wider."""
+    from moldy_amd import system
+    s = system.water_box(n, seed=3, alpha=alpha, cutoff=14.0)
+    s.h = s.h * widen
+    s.c_of_m = s.c_of_m / widen
+    return s
+
+
+def test_systems_of_these_tests_take_the_grid():
+    from moldy_amd import engine as E, system
+    for name in ("water", "skewed", "salt", "silica"):
+        assert _route(_system(name), E.FP64), name
+    for name in ("skewed", "salt", "silica"):
+        assert _route(_system(name), E.MIXED), name
+    for prec in (E.FP64, E.MIXED):
+        assert _route(_past_rule(prec), prec)
+    assert _route(system.salt_water(nwater=2800, nmg=50, ncl=100, seed=13), E.FP64)
+    assert _route(system.salt_water(nwater=4200, nmg=76, ncl=152, seed=13), E.MIXED)
+    # test_gpu_adjoint_grid.py's FP64 sides, and the replayed MD step's mixed one
+    assert _route(system.water_box(3600, seed=31), E.FP64)
+    assert _route(system.silica(ncell=7, seed=32, cutoff=10.0), E.FP64)
+    assert _route(system.water_box(5000, seed=23), E.MIXED)
+
+
+def test_full_bricks_of_a_droplet():
+    """Bricks of 126 sites beside empty ones (the mean is 4): within the bucket
+    that a dense liquid fills."""
+    from moldy_amd import engine as E
+    from oracle.oracle import Oracle
+    s = _droplet(4000, 3.0, 0.15)
+    assert _route(s, E.FP64)
+    _check(s, Oracle(s).make_sites(), E.FP64, 1e-11, 5e-11)
