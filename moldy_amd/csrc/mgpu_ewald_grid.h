@@ -40,7 +40,6 @@ GridGeom grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const double h
                    double alpha, double kc, bool fp64);
 // Whether the gridded sum takes this system (it can, and it pays).
 bool grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const std::vector<KRow> &rows);
-bool grid_pays(const GridGeom &g, int nk);
 GridSizes grid_sizes(const GridGeom &g);
 void grid_tables(const GridGeom &g, GridTables &t);
 void grid_rowmap(const GridGeom &g, const std::vector<KRow> &rows, std::vector<int> &map);

@@ -871,6 +871,33 @@ GridGeom mgpu::grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const do
    return g;
 }
 
+namespace {
+// Where the grid beats the direct sum: its thirteen launches cost a floor that
+// N_k N_s products must outweigh, its transforms depend on the grid alone, and
+// with coarse points a tile of them holds so many sites that few blocks do the
+// spreading and gathering.  MD step, direct against grid, us:
+//   products    FP64 8,800 water sites (5.4e7) 216 and 226, 10,800 (8.2e7) 314 and 285,
+//               16,384 (1.9e8) 344 and 256, 132,872 salt water (1.3e10) 7,870 and 1,112; mixed 14,400
+//               water (1.5e8) 171 and 174, 12,288 silica (2.2e8) 166 and 157, 32,000 water
+//               (7.2e8) 254 and 215, 132,872 1,336 and 635
+//   transforms  few sites in a wide box or at a high cutoff: mixed 700 sites, 6.6e9
+//               multiply-adds, 3.4e8 products 265 and 514, 4,000, 6e8, 3e8 184 and 199, 8,000, 2.7e8,
+//               3.6e8 181 and 190, 16,000, 3e8, 5.4e8 203 and 196.  The FP64 direct sum slows as the
+//               transforms grow: 700, 1.4e9, 8.1e7 310 and 298, 9.6e9, 3.4e8 4,184 and 887, 2,400,
+//               4.5e8, 1.1e8 224 and 238, 8,000, 3.8e8, 3.6e8 365 and 272: no term
+//   points      alpha 0.15 (FP64 1.8 A^3 a point, mixed 2.8): a droplet of 16,000 sites, 1.8e8
+//               products, FP64 367 and 420, 6.1e8 mixed 244 and 309; 80,000 sites, 1.9e9 mixed 559 and 500
+bool grid_pays(const GridGeom &g, int nk) {
+   const double direct = (double)nk * g.ns, L = g.m[2] + 1;
+   double points = 1;
+   for (int d = 0; d < 3; d++) points *= g.n[d];
+   const double macs = 2 * (points * 2 * L + 4.0 * g.n[0] * g.n[1] * (g.m[1] + 1) * L +
+                            4.0 * g.n[0] * (g.m[0] + 1) * (2 * g.m[1] + 1) * L);
+   const double coarse = g.vol / points / (g.fp64 ? 0.45 : 0.69);
+   return direct > (g.fp64 ? 8e7 : std::max(2e8, 1e8 + macs)) * std::max(1.0, coarse);
+}
+}  // namespace
+
 bool mgpu::grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const std::vector<KRow> &rows) {
    // frameworks need two structure factors a k; the window's width counts on
    // the Gaussian damping of the last k; one row per (h, k) is the reference's set
@@ -881,17 +908,6 @@ bool mgpu::grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const st
    for (int d = 0; d < 3; d++)
       if (g.n[d] > 512 || g.n[d] < 4 * g.m[d]) return false;
    return grid_pays(g, nk);
-}
-
-// Where the grid beats the direct sum: its thirteen launches and its small
-// transforms cost a floor that N_k N_s products must outweigh.  MD step, direct
-// against grid: FP64 5,184 silica sites (3.8e7 products) 190 and 183 us, 8,800 water
-// sites (5.4e7) 216 and 226, 16,384 (1.9e8) 344 and 256, 132,872 salt water (1.3e10)
-// 7,870 and 1,112; mixed 16,384 water sites 184 and 193 us, 12,288 silica sites
-// (2.2e8) 191 and 181, 32,000 water (7.2e8) 290 and 237, 132,872 1,336 and 635.
-bool mgpu::grid_pays(const GridGeom &g, int nk) {
-   const double direct = (double)nk * g.ns;
-   return direct > (g.fp64 ? 8e7 : 2e8);
 }
 
 GridSizes mgpu::grid_sizes(const GridGeom &g) {

@@ -246,3 +246,57 @@ def test_full_bricks_of_a_droplet():
     s = _droplet(4000, 3.0, 0.15)
     assert _route(s, E.FP64)
     _check(s, Oracle(s).make_sites(), E.FP64, 1e-11, 5e-11)
+
+
+@pytest.mark.parametrize("kind,prec,grid", [
+    ("few sites, high cutoff", 1, False),     # 700 sites, a grid of 248^3
+    ("few sites, high cutoff", 0, True),
+    ("wide box", 1, False),                   # 4,000 sites in nine times their volume
+    ("coarse droplet", 1, False),
+    ("coarse liquid", 1, False),
+    ("slab", 1, True),
+])
+def test_size_rule(kind, prec, grid):
+    from moldy_amd import system
+    if kind == "few sites, high cutoff":
+        s = system.water_box(175, seed=3, alpha=3.0, cutoff=6.0)
+    elif kind == "wide box":
+        s = system.water_box(1000, seed=3)
+        s.h = s.h * 3.0
+    elif kind == "coarse droplet":
+        s = _droplet(4000, 3.0, 0.15)
+    elif kind == "coarse liquid":
+        s = system.water_box(16000, seed=3, alpha=0.15, cutoff=18.0)
+    else:
+        s = system.water_box(8000, seed=3)
+        s.h = s.h * np.array([1.0, 1.0, 3.0])
+        s.c_of_m = s.c_of_m / np.array([1.0, 1.0, 3.0])
+    assert _route(s, prec) == grid
+
+
+def _flat(thin, order):
+    """Water on a jittered 5 x 35 x 36 lattice, its thin side (24 grid points: three
+    bricks, the fewest) along axis thin; 21 and 22 bricks (FP64), 18 and 19 (mixed)
+    along the others."""
+    from moldy_amd import system
+    n = np.array(order)
+    a = 2.9
+    s = system.water_box(int(np.prod(n)), seed=9, cutoff=6.0)
+    rng = np.random.default_rng(9)
+    grid = np.stack(np.meshgrid(*[np.arange(k) for k in n], indexing="ij"), -1).reshape(-1, 3)
+    pos = (grid + 0.5) / n - 0.5 + rng.normal(0, 0.1 / (a * n), grid.shape)
+    s.c_of_m = pos - np.floor(pos + 0.5)
+    s.h = np.diag(a * n)
+    assert n[thin] == 5
+    return s
+
+
+@pytest.mark.parametrize("thin,order", [(0, (5, 35, 36)), (1, (36, 5, 35)), (2, (35, 36, 5))])
+def test_flat_box(thin, order):
+    from moldy_amd import engine as E
+    from oracle.oracle import Oracle
+    s = _flat(thin, order)
+    xyz = Oracle(s).make_sites()
+    for prec, tol in ((E.FP64, (1e-11, 5e-11)), (E.MIXED, (2e-6, 1e-6))):
+        assert _route(s, prec)
+        _check(s, xyz, prec, *tol)
