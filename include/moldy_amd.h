@@ -119,15 +119,20 @@ int mgpu_ewald(mgpu_engine *eng, const double h[9], const double *site, int ld,
  * No counterpart in the reference.  For callers that cannot allocate
  * device memory (code under stream capture, tight serving loops, harnesses
  * that forbid hipMalloc): the arguments, semantics and results of
- * mgpu_ewald, FP64 only, with every device buffer it needs -- copies of
- * site, chg and site_force, the k rows, trig tables, structure-factor
- * partials, weights and back-projection partials -- taken from one static
- * array of MGPU_NOALLOC_BYTES (64 MiB) that each GPU holds from the
- * engine's creation until the process ends.  The call makes no allocation
- * of any kind; a system whose buffers do not fit returns MGPU_E_CAPACITY
- * with the size it needs.  Calls on one GPU share its array: calls that
- * overlap in time on one GPU race.  Results are bit-identical to
- * mgpu_ewald's (the same kernels, launch shapes and summation order). */
+ * mgpu_ewald, FP64 only, with every device buffer it needs taken from one
+ * static array of MGPU_NOALLOC_BYTES (64 MiB) that each GPU holds from the
+ * engine's creation until the process ends: copies of site, chg and
+ * site_force, the k rows, and for the direct sum trig tables,
+ * structure-factor partials, weights and back-projection partials, for the
+ * gridded sum its grid, half-transformed modes, the sites' window weights and
+ * the transforms' tables.  The call makes no device allocation (host memory
+ * for the k set and the tables is the usual heap's); a system whose buffers
+ * do not fit returns MGPU_E_CAPACITY with the size it needs.  Calls on one
+ * GPU share its array: calls that overlap in time on one GPU race.  Results
+ * are bit-identical to mgpu_ewald's (the same kernels, launch shapes and
+ * summation order), except where mgpu_ewald takes the gridded sum and only
+ * the direct sum's buffers fit: then the direct sum runs, and the two agree
+ * to rounding. */
 int mgpu_ewald_noalloc(mgpu_engine *eng, const double h[9], const double *site, int ld,
                        const double *chg, double *site_force, double *pe, double stress[9],
                        mgpu_ew_info *info);

@@ -837,43 +837,59 @@ void mgpu::ewald_noalloc(mgpu_engine *e, const double h[9], const double *site, 
    g.hmax = ks.hmax; g.kmax = ks.kmax; g.lmax = ks.lmax;
    g.vol = host_det(h);
    g.alpha = e->alpha;
-   // the same choice of sum as mgpu_ewald's
+   // the same choice of sum as mgpu_ewald's, unless only the direct sum's buffers fit
    const GridGeom gg = grid_geom(g.ns, g.nsp, g.hmax, g.kmax, g.lmax, h, g.hinv, g.vol, g.alpha, e->k_cutoff, true);
-   const bool grid = grid_applies(gg, g.nsxf, g.nk, e->k_cutoff, ks.rows);
-   GridTables gt;
+   const GridSizes gz = grid_sizes(gg);
+   bool grid = gz.bytes <= (size_t)MGPU_NOALLOC_BYTES && grid_applies(gg, g.nsxf, g.nk, e->k_cutoff, ks.rows);
+   std::shared_ptr<const GridTables> gt;
    std::vector<int> gmap;
    if (grid) {
-      grid_tables(gg, gt);
+      gt = grid_host_tables(e, gg);
       grid_rowmap(gg, ks.rows, gmap);
    }
-   const GridSizes gz = grid_sizes(gg);
    const Ew64Sizes z = ew64_sizes(g, e->ncu, npart);
-   // carve the regions, 256-byte aligned
-   size_t off = 0;
-   auto take = [&](size_t bytes) {
-      const size_t o = off;
-      off += (bytes + 255) & ~(size_t)255;
-      return o;
-   };
+   // the regions, 256-byte aligned
    const size_t nsp = g.nsp;
-   const size_t oSite = take(sizeof(double) * 3 * nsp), oForce = take(sizeof(double) * 3 * nsp),
-                oChg = chg ? take(sizeof(double) * nsp) : 0, oRows = take(sizeof(KRow) * (g.nrows + 1)),
-                oOut = take(sizeof(double) * 8);
-   size_t oKrow = 0, oRpart = 0, oTx = 0, oTy = 0, oTz = 0, oSk = 0, oWk = 0, oRed = 0, oFpart = 0, oZt = 0, oW64 = 0,
-          oGrid = 0, oGtab = 0, oGmap = 0;
-   if (grid) {
-      oGrid = take(gz.bytes);
-      oGtab = take(sizeof(double) * gt.data.size());
-      oGmap = take(sizeof(int) * gmap.size());
-   } else {
-      oKrow = take(sizeof(int) * (g.nk + 1)), oRpart = take(sizeof(int) * (npart + 1)),
-      oTx = take(sizeof(double2) * z.tx), oTy = take(sizeof(double2) * z.ty), oTz = take(sizeof(double2) * z.tz),
-      oSk = take(sizeof(double) * z.sk), oWk = take(sizeof(double) * z.wk), oRed = take(sizeof(double) * z.red),
-      oFpart = take(sizeof(double) * z.fpart), oZt = take(sizeof(double) * z.zt64),
-      oW64 = take(sizeof(double) * z.w64);
+   size_t off = 0, oSite, oForce, oChg, oRows, oOut, oRtmp, oKrow = 0, oRpart = 0, oTx = 0, oTy = 0, oTz = 0, oSk = 0,
+          oWk = 0, oRed = 0, oFpart = 0, oZt = 0, oW64 = 0, oGrid = 0, oGtab = 0, oGmap = 0;
+   int nred = 0;
+   auto carve = [&] {
+      off = 0;
+      auto take = [&](size_t bytes) {
+         const size_t o = off;
+         off += (bytes + 255) & ~(size_t)255;
+         return o;
+      };
+      oSite = take(sizeof(double) * 3 * nsp);
+      oForce = take(sizeof(double) * 3 * nsp);
+      oChg = chg ? take(sizeof(double) * nsp) : 0;
+      oRows = take(sizeof(KRow) * (g.nrows + 1));
+      oOut = take(sizeof(double) * 8);
+      if (grid) {
+         oGrid = take(gz.bytes);
+         oGtab = take(sizeof(double) * gt->data.size());
+         oGmap = take(sizeof(int) * gmap.size());
+      } else {
+         oKrow = take(sizeof(int) * (g.nk + 1));
+         oRpart = take(sizeof(int) * (npart + 1));
+         oTx = take(sizeof(double2) * z.tx);
+         oTy = take(sizeof(double2) * z.ty);
+         oTz = take(sizeof(double2) * z.tz);
+         oSk = take(sizeof(double) * z.sk);
+         oWk = take(sizeof(double) * z.wk);
+         oRed = take(sizeof(double) * z.red);
+         oFpart = take(sizeof(double) * z.fpart);
+         oZt = take(sizeof(double) * z.zt64);
+         oW64 = take(sizeof(double) * z.w64);
+      }
+      nred = grid ? gz.nred : z.nkb;
+      oRtmp = take(sizeof(double) * ((size_t)reduce_cols_blocks(nred) * 8 + 17));
+   };
+   carve();
+   if (grid && off > (size_t)MGPU_NOALLOC_BYTES) {
+      grid = false;
+      carve();
    }
-   const int nred = grid ? gz.nred : z.nkb;
-   const size_t oRtmp = take(sizeof(double) * ((size_t)reduce_cols_blocks(nred) * 8 + 17));
    if (off > (size_t)MGPU_NOALLOC_BYTES)
       throw StatusError{MGPU_E_CAPACITY, "mgpu_ewald_noalloc: this system needs " + std::to_string(off >> 20) +
                                              " MiB of scratch; the limit is " +
@@ -904,13 +920,13 @@ void mgpu::ewald_noalloc(mgpu_engine *e, const double h[9], const double *site, 
    if (chg) HIPCHK(hipMemcpyAsync(base + oChg, chg, sizeof(double) * g.ns, hipMemcpyHostToDevice, st));
    HIPCHK(hipMemcpyAsync(base + oRows, ks.rows.data(), sizeof(KRow) * g.nrows, hipMemcpyHostToDevice, st));
    if (grid) {
-      HIPCHK(hipMemcpyAsync(base + oGtab, gt.data.data(), sizeof(double) * gt.data.size(), hipMemcpyHostToDevice, st));
+      HIPCHK(hipMemcpyAsync(base + oGtab, gt->data.data(), sizeof(double) * gt->data.size(), hipMemcpyHostToDevice, st));
       HIPCHK(hipMemcpyAsync(base + oGmap, gmap.data(), sizeof(int) * gmap.size(), hipMemcpyHostToDevice, st));
       grid_clear(e, gg, base + oGrid);
       GridBufs gb;
       gb.site = dsite; gb.w = b.w; gb.force = b.force; gb.rows = b.rows; gb.rowmap = (const int *)(base + oGmap);
       gb.tab = (const double *)(base + oGtab); gb.base = base + oGrid; gb.prof = false;
-      grid_pass(e, nullptr, gg, gt, gb, false);
+      grid_pass(e, nullptr, gg, *gt, gb, false);
       reduce_cols_into(nullptr, st, (const double *)(base + oGrid + gz.bpart), nred, 8, b.out, b.rtmp, b.count);
    } else {
       HIPCHK(hipMemcpyAsync(base + oKrow, ks.krow.data(), sizeof(int) * g.nk, hipMemcpyHostToDevice, st));

@@ -42,6 +42,10 @@ GridGeom grid_geom(int ns, int nsp, int hmax, int kmax, int lmax, const double h
 bool grid_applies(const GridGeom &g, int nsxf, int nk, double kc, const std::vector<KRow> &rows);
 GridSizes grid_sizes(const GridGeom &g);
 void grid_tables(const GridGeom &g, GridTables &t);
+// The host tables for g: the engine's plan's where they are the same, else kept
+// on the engine from one call to the next (mgpu_ewald_noalloc: building them
+// takes 0.14 ms at 72 points an axis, 0.7 ms at 168).
+std::shared_ptr<const GridTables> grid_host_tables(mgpu_engine *e, const GridGeom &g);
 void grid_rowmap(const GridGeom &g, const std::vector<KRow> &rows, std::vector<int> &map);
 // Clears what a pass expects cleared (brick counts); a
 // pass leaves it so.

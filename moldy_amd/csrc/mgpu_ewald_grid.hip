@@ -1246,6 +1246,30 @@ void mgpu::grid_clear(mgpu_engine *e, const GridGeom &g, uint8_t *base) {
    zero_async(e, base + z.cnt, 4 * (size_t)g.nb[0] * g.nb[1] * g.nb[2]);
 }
 
+// What the tables and the place of the brick counts depend on.
+static void table_key(const GridGeom &g, int key[8]) {
+   for (int d = 0; d < 3; d++) {
+      key[d] = g.n[d];
+      key[3 + d] = g.m[d];
+   }
+   key[6] = g.fp64;
+   key[7] = g.ns;
+}
+
+std::shared_ptr<const GridTables> mgpu::grid_host_tables(mgpu_engine *e, const GridGeom &g) {
+   int key[8];
+   table_key(g, key);
+   if (e->grid_tab && memcmp(key, e->grid_key, sizeof key) == 0) return e->grid_tab;
+   if (!e->grid_host_tab || memcmp(key, e->grid_host_key, sizeof key) != 0) {
+      e->grid_host_tab.reset();
+      auto t = std::make_shared<GridTables>();
+      grid_tables(g, *t);
+      e->grid_host_tab = t;
+      memcpy(e->grid_host_key, key, sizeof key);
+   }
+   return e->grid_host_tab;
+}
+
 // The engine's plan for its geometry and precision, made where it is missing
 // or stale; false where the direct sum is to run.
 static bool grid_plan(mgpu_engine *e, GridGeom &g) {
@@ -1256,7 +1280,8 @@ static bool grid_plan(mgpu_engine *e, GridGeom &g) {
    const GridSizes z = grid_sizes(g);
    // the plan: tables of the grid's sizes, the k set's row map, and the
    // cleared parts of the scratch block
-   const int key[8] = {g.n[0], g.n[1], g.n[2], g.m[0], g.m[1], g.m[2], fp64, g.ns};
+   int key[8];
+   table_key(g, key);
    const bool same = e->grid_tab && memcmp(key, e->grid_key, sizeof key) == 0;
    if (e->capturing && (!same || e->grid_version != e->geom_version))
       throw StatusError{MGPU_E_STATE, "gridded Ewald plan changed during capture"};

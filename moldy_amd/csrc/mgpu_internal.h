@@ -224,6 +224,8 @@ struct mgpu_engine {
    // |h| |k| |l|, FP64, sites), the k set's row map, scratch
    std::shared_ptr<const mgpu::GridTables> grid_tab;
    int grid_key[8] = {0};
+   std::shared_ptr<const mgpu::GridTables> grid_host_tab;   // mgpu_ewald_noalloc's
+   int grid_host_key[8] = {0};
    int grid_version = -1;
    mgpu::DBuf<double> d_gtab;
    mgpu::DBuf<uint8_t> d_grid;

@@ -274,6 +274,31 @@ def test_size_rule(kind, prec, grid):
     assert _route(s, prec) == grid
 
 
+@pytest.mark.parametrize("nwater,hmax", [(375, 36), (200, 40)])
+def test_noalloc_takes_the_direct_sum_where_only_that_fits(nwater, hmax):
+    """Few sites at a high cutoff: the grid needs 65 and 95 MiB, the direct sum 37
+    and 48 of the 64."""
+    from moldy_amd import engine as E, system
+    from oracle.oracle import Oracle
+    import test_zz_no_alloc as T
+    s = system.water_box(nwater, seed=3, cutoff=6.0)
+    s.control.k_cutoff = 2 * np.pi * (hmax + 0.5) / s.h[0, 0]
+    s.control.alpha = s.control.k_cutoff / (2 * np.sqrt(-np.log(1e-6)))
+    assert _route(s, E.FP64)
+    xyz = Oracle(s).make_sites()
+    f0 = np.random.default_rng(3).standard_normal((3, s.nsites))
+    e = E.ForceEngine(s)
+    rc, fa, pa, sa, ia = T._call(e, "mgpu_ewald_noalloc", s, xyz, f0)
+    assert rc == 0, E.lib().mgpu_last_error(e.h_)
+    rc, fb, pb, sb, ib = T._call(e, "mgpu_ewald", s, xyz, f0)
+    assert rc == 0 and ia.hmax == ib.hmax == hmax
+    e.close()
+    # two sums of the same terms
+    assert rel_err(fa - f0, fb - f0) < 1e-11
+    assert abs(pa - pb) <= 5e-11 * (abs(pb) + ia.self_energy)
+    assert rel_err(sa, sb) < 5e-11
+
+
 def _flat(thin, order):
     """Water on a jittered 5 x 35 x 36 lattice, its thin side (24 grid points: three
     bricks, the fewest) along axis thin; 21 and 22 bricks (FP64), 18 and 19 (mixed)
