@@ -423,10 +423,14 @@ def main():
                            alpha_per_A=0.30, k_cutoff_per_A=round(s.control.k_cutoff, 4),
                            cells=[fc.nx, fc.ny, fc.nz], dt_fs=DT_FS,
                            precision=a.precision))
-    res["autotuned_shapes"] = {"fp64": dict(fp64_backprojection_parts=tuned["fp64"][1])}
-    if "mixed" in tuned:
-        res["autotuned_shapes"]["mixed"] = dict(sk_workgroups=tuned["mixed"][0],
-                                                backprojection_rounds=tuned["mixed"][1])
+    # launch shapes of the direct reciprocal sum (the gridded sum has none)
+    shapes = {}
+    if "ewald_force" in prof64:
+        shapes["fp64"] = dict(fp64_backprojection_parts=tuned["fp64"][1])
+    if mixed and "ewald_mfma_force" in mixed["prof"]:
+        shapes["mixed"] = dict(sk_workgroups=tuned["mixed"][0], backprojection_rounds=tuned["mixed"][1])
+    if shapes:
+        res["autotuned_shapes"] = shapes
     res["fp64_evals_per_s"] = 1.0 / t64
     res["fp64_ms_per_eval"] = 1e3 * t64
     if mixed:

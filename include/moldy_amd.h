@@ -269,8 +269,9 @@ int mgpu_adjoint(mgpu_engine *eng, const double *v, const double *dtheta, double
  * the S(k) MFMA workgroup count and the MFMA back-projection grid (mixed;
  * returned in sk_blocks and npart: 0 = one workgroup per 128-site block,
  * r > 0 = r rounds of resident workgroups sharing the work equally), or the
- * FP64 back-projection row partitions (npart); results are identical up to
- * the order of partial sums. */
+ * FP64 back-projection row partitions (npart); both 0 where the evaluation
+ * takes the gridded sum, which has no such shape (the overlap is tuned all
+ * the same).  Results are identical up to the order of partial sums. */
 enum { MGPU_SCHED_GRAPH = 0, MGPU_SCHED_STREAM_GRAPHS = 1, MGPU_SCHED_STREAMS = 2, MGPU_SCHED_GROUPED = 3 };
 typedef struct mgpu_batch mgpu_batch;
 int  mgpu_batch_create(mgpu_batch **batch, int device);

@@ -431,25 +431,30 @@ void finish(mgpu_batch *b, int nsteps, double *trace) {
    }
 }
 
-// Process-wide memory of tuned shapes: (precision, nrows, lmax, nsites/4096)
-// -> (S(k) workgroups, MFMA back-projection partitions, FP64 partitions).
-std::map<std::tuple<int, int, int, int>, std::array<int, 4>> g_tuned;
+// Process-wide memory of tuned shapes: (precision, nrows, lmax, nsites/4096,
+// gridded sum) -> (S(k) workgroups, MFMA back-projection partitions, FP64
+// partitions, overlap).
+std::map<std::tuple<int, int, int, int, bool>, std::array<int, 4>> g_tuned;
 
 }  // namespace
 
 // Time the tunable launch shapes of e's force evaluation and keep the
 // fastest: the S(k) workgroup count and the back-projection row partitions
 // of the MFMA Ewald (mixed precision), or the row partitions of the FP64
-// back-projection.  Results are identical up to the summation order of
-// partial sums.
+// back-projection; none of these where the gridded sum runs, which has no such
+// shape (only the overlap is tuned then).  Results are identical up to the
+// summation order of partial sums.
 void mgpu::autotune_engine(mgpu_engine *e, int reps, int *sk_blocks, int *npart) {
    if (e->alpha <= 1e-7) return;
-   auto key = std::make_tuple(e->precision, e->nrows, e->lmax, e->nsites / 4096);
+   const bool grid = grid_chosen(e);
+   auto key = std::make_tuple(e->precision, e->nrows, e->lmax, e->nsites / 4096, grid);
    auto it = g_tuned.find(key);
    if (it != g_tuned.end()) {
-      e->tune_sk_blocks = it->second[0];
-      e->tune_force_parts = it->second[1];
-      e->tune_npart = it->second[2];
+      if (!grid) {
+         e->tune_sk_blocks = it->second[0];
+         e->tune_force_parts = it->second[1];
+         e->tune_npart = it->second[2];
+      }
       e->overlap = it->second[3];
    } else {
       hipEvent_t t0, t1;
@@ -482,11 +487,11 @@ void mgpu::autotune_engine(mgpu_engine *e, int reps, int *sk_blocks, int *npart)
             }
          field = cand[std::min_element(t.begin(), t.end()) - t.begin()];
       };
-      if (e->precision == MGPU_MIXED) {
+      if (!grid && e->precision == MGPU_MIXED) {
          const int slots = e->ncu;   // one S(k) workgroup per CU (LDS)
          tune(e->tune_sk_blocks, {2 * slots, 3 * slots, 4 * slots, 6 * slots, 8 * slots, 12 * slots});
          tune(e->tune_force_parts, {0, 1, 2, 4});
-      } else {
+      } else if (!grid) {
          tune(e->tune_npart, {4, 8, 16, 32});
       }
       // real space beside the Ewald sum, or after it: a difference of a few
@@ -499,8 +504,8 @@ void mgpu::autotune_engine(mgpu_engine *e, int reps, int *sk_blocks, int *npart)
       g_tuned[key] = {e->tune_sk_blocks, e->tune_force_parts, e->tune_npart, e->overlap};
    }
    e->geom_version++;
-   if (sk_blocks) *sk_blocks = e->precision == MGPU_MIXED ? e->tune_sk_blocks : 0;
-   if (npart) *npart = e->precision == MGPU_MIXED ? e->tune_force_parts : e->tune_npart;
+   if (sk_blocks) *sk_blocks = !grid && e->precision == MGPU_MIXED ? e->tune_sk_blocks : 0;
+   if (npart) *npart = grid ? 0 : e->precision == MGPU_MIXED ? e->tune_force_parts : e->tune_npart;
 }
 
 extern "C" {

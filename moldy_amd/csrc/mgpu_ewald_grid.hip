@@ -1270,13 +1270,22 @@ std::shared_ptr<const GridTables> mgpu::grid_host_tables(mgpu_engine *e, const G
    return e->grid_host_tab;
 }
 
+// The grid of the engine's geometry and precision; whether it is to be used.
+static bool engine_grid(const mgpu_engine *e, GridGeom &g) {
+   g = grid_geom(e->nsites, e->nsp, e->hmax, e->kmax, e->lmax, e->h, e->hinv, host_det(e->h), e->alpha, e->k_cutoff,
+                 e->precision == MGPU_FP64);
+   return grid_applies(g, e->nsitesxf, e->nk, e->k_cutoff, e->rows);
+}
+
+bool mgpu::grid_chosen(const mgpu_engine *e) {
+   GridGeom g;
+   return engine_grid(e, g);
+}
+
 // The engine's plan for its geometry and precision, made where it is missing
 // or stale; false where the direct sum is to run.
 static bool grid_plan(mgpu_engine *e, GridGeom &g) {
-   const bool fp64 = e->precision == MGPU_FP64;
-   g = grid_geom(e->nsites, e->nsp, e->hmax, e->kmax, e->lmax, e->h, e->hinv, host_det(e->h),
-                                e->alpha, e->k_cutoff, fp64);
-   if (!grid_applies(g, e->nsitesxf, e->nk, e->k_cutoff, e->rows)) return false;
+   if (!engine_grid(e, g)) return false;
    const GridSizes z = grid_sizes(g);
    // the plan: tables of the grid's sizes, the k set's row map, and the
    // cleared parts of the scratch block

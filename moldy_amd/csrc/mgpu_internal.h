@@ -318,6 +318,7 @@ void run_rdf(mgpu_engine *e, double limit, int nbins, int noff, float *rdf_host)
 void run_ewald_fp64(mgpu_engine *e);        // -> d_out[OUT_RECIP..]
 void run_ewald_mixed(mgpu_engine *e);       // -> d_out[OUT_RECIP..]
 bool run_ewald_grid(mgpu_engine *e);        // the same; false (nothing done) where the direct sum is to run
+bool grid_chosen(const mgpu_engine *e);     // whether run_ewald_grid runs it
 // The device part of eval_forces after the two boundary calls: second
 // make_sites, dipole and surface term, molecular forces and torques, virial
 // correction and the assembly of pe, dipole and stress into d_out[OUT_RES..].

@@ -126,3 +126,28 @@ def test_autotune():
     b.close()
     for e in eng:
         e.close()
+
+
+def test_autotune_beside_the_gridded_sum():
+    """The gridded sum has no shapes to tune; a system of the same k rows and size
+    class on the direct side of the size rule is tuned by itself, not given the
+    shapes of one that never ran them."""
+    from moldy_amd import engine as E, system
+    s = system.water_box(2700, seed=3)          # 10,800 sites, 8.2e7 products: gridded
+    d = s.copy()
+    d.species = [system.water_species(2500)]    # 7.6e7: direct, the same box
+    d.c_of_m, d.quat = s.c_of_m[:2500].copy(), s.quat[:2500].copy()
+    assert s.nsites // 4096 == d.nsites // 4096
+    out = []
+    for x in (s, d):
+        e = E.ForceEngine(x)
+        e.upload_state()
+        e.profile(True)
+        pe = e.eval_forces_device()[0].copy()
+        grid = e.profile_get("ewald_grid_spread")[1] > 0
+        shape = e.autotune()
+        assert np.allclose(e.eval_forces_device()[0], pe, rtol=1e-12, atol=0)
+        out.append((grid, shape))
+        e.close()
+    assert out[0] == (True, (0, 0))
+    assert out[1][0] is False and out[1][1][0] == 0 and out[1][1][1] in (4, 8, 16, 32)
