@@ -1123,21 +1123,21 @@ void mgpu::ewald_charge_adjoint(mgpu_engine *e, const double *v, const double *d
    ewald_plan(e);
    const int nk = e->nk, nid = e->max_id, nsp = e->nsp, ns = e->nsites;
    const int nb = (nsp + 255) / 256;
-   // scratch: coeff/k, C+iS for q, each id, q v_x..z, direction; phi; weights
+   // scratch: coeff/k, C+iS for q, each id, q v_x..z, direction; phi; weights;
+   // partial sums and the sums per id
    size_t off = 0;
    auto take = [&](size_t bytes) { size_t o = off; off += (bytes + 255) & ~(size_t)255; return o; };
    const size_t oKc = take(sizeof(double4) * nk), oQ = take(sizeof(double2) * nk),
                 oA = take(sizeof(double2) * nk * (size_t)nid), oV = take(sizeof(double2) * nk * 3),
                 oD = take(sizeof(double2) * nk), oPhi = take(sizeof(double) * 3 * nsp),
-                oW = take(sizeof(double) * nsp), oP = take(sizeof(double) * (size_t)std::max(nk, nsp) / 256 * 2 * nid + 64 * nid);
+                oW = take(sizeof(double) * nsp), oP = take(sizeof(double) * (size_t)std::max(nk, nsp) / 256 * 2 * nid + 64 * nid),
+                oO = take(sizeof(double) * 2 * nid);
    e->d_adj.reserve(off);
    uint8_t *B = e->d_adj.p;
    double4 *kc = (double4 *)(B + oKc);
    double2 *csq = (double2 *)(B + oQ), *csa = (double2 *)(B + oA), *csv = (double2 *)(B + oV),
            *csd = (double2 *)(B + oD);
-   double *phi = (double *)(B + oPhi), *w = (double *)(B + oW), *part = (double *)(B + oP);
-   e->d_out.reserve(OUT_SIZE);
-   double *outc = e->d_out.p + OUT_TMP;
+   double *phi = (double *)(B + oPhi), *w = (double *)(B + oW), *part = (double *)(B + oP), *outc = (double *)(B + oO);
    KcArgs ka{nk, host_det(e->h), -1.0 / (4.0 * e->alpha * e->alpha), 2 * PI_D * e->hinv[8], e->d_rows.p, e->d_krow.p};
    k_kcoeff<<<(nk + 255) / 256, 256, 0, e->stream>>>(ka, kc);
    weighted_sf(e, e->d_chg_site.p, csq);

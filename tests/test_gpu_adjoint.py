@@ -164,3 +164,43 @@ def test_force_matching_gradient_through_autograd():
     print(f"force matching: |grad| {np.abs(fd).max():.3e}  rel err {err:.1e}")
     assert err < TOL
     fw.eng.close()
+
+
+def test_sixteen_ids():
+    """Ten more ids without sites (the most an engine takes): every derivative as
+    without them, zeros for theirs."""
+    from moldy_amd import engine as E, system
+    s = S.salt()
+    n = 16
+    big = s.copy()
+    big.potpar = system.empty_potpar(n)
+    big.potpar[:s.max_id, :s.max_id] = s.potpar
+    big.site_mass = np.concatenate([s.site_mass, np.zeros(n - len(s.site_mass))])
+    big.site_charge = np.concatenate([s.site_charge, np.zeros(n - s.max_id)])
+    assert big.max_id == n
+    npar = s.n_potpar
+    pairs = [(a, b) for a in range(n) for b in range(a, n)]
+    old = [(a, b) for a in range(s.max_id) for b in range(a, s.max_id)]
+    at = [pairs.index(p) * npar + k for p in old for k in range(npar)]
+    at += [len(pairs) * npar + a for a in range(s.max_id)]
+    rng = np.random.default_rng(4)
+    v = rng.standard_normal((3, s.nsites))
+    th = E.get_theta(s)
+    d = rng.standard_normal(th.size) * np.abs(th)
+    dbig = np.zeros(E.get_theta(big).size)
+    dbig[at] = d
+    out = []
+    for x, dt in ((s, d), (big, dbig)):
+        e = E.ForceEngine(x)
+        e.upload_state()
+        out.append(e.adjoint(v=v, dtheta=dt))
+        e.close()
+    a, b = out
+    rest = np.setdiff1d(np.arange(dbig.size), at)
+    for k in ("dE", "vjp"):
+        # sums over the waves' sites, cut differently: few eps of their terms
+        assert np.linalg.norm(b[k][at] - a[k]) <= 1e-11 * np.linalg.norm(a[k])
+        q = slice(-s.max_id, None)
+        assert np.allclose(b[k][at][q], a[k][q], rtol=1e-9, atol=1e-11 * np.abs(a[k][q]).max())
+        assert np.all(b[k][rest] == 0.0)
+    assert np.linalg.norm(b["jvp"] - a["jvp"]) <= 1e-11 * np.linalg.norm(a["jvp"])
