@@ -358,10 +358,13 @@ void enqueue_steps(mgpu_batch *b, int nsteps, bool init_h0, int s) {
       zero_async(e, e->d_iflags.p, sizeof(int) * 48);
    }
    if (nsteps <= 0) return;
-   // The first step runs eagerly (it makes every buffer) unless the
-   // schedule's captured step is current: then every step is a replay.
-   const bool replay_all =
-       (s == MGPU_SCHED_GROUPED && !grouped_stale(b)) || (s == MGPU_SCHED_GRAPH && !graph_stale(b));
+   // The first step runs eagerly (it makes every buffer, and is what a profile
+   // times) unless the schedule's captured step is current: then every step
+   // is a replay.
+   bool prof = false;
+   for (auto *e : b->eng) prof = prof || e->prof_on;
+   const bool replay_all = !prof && ((s == MGPU_SCHED_GROUPED && !grouped_stale(b)) ||
+                                     (s == MGPU_SCHED_GRAPH && !graph_stale(b)));
    const int first = replay_all ? 0 : 1;
    if (!replay_all) {
       for (auto *e : b->eng) md_step_launch(e);

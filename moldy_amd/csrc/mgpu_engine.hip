@@ -1188,10 +1188,11 @@ int mgpu_md_steps(mgpu_engine *e, int nsteps, int init_h0, int use_graph, double
          }
          e->cell_valid = true;
       } else {
-         // the first step runs eagerly (it makes every buffer) unless the
-         // captured step is current: then every step is a replay
+         // the first step runs eagerly (it makes every buffer, and is what a
+         // profile times) unless the captured step is current: then every step
+         // is a replay
          int done = 0;
-         if (!use_graph || !step_graph_current(e)) {
+         if (!use_graph || e->prof_on || !step_graph_current(e)) {
             md_step_launch(e);
             done = 1;
          }

@@ -46,6 +46,32 @@ def test_replayed_first_step_is_bitwise_eager(prec, nvt):
     e.close()
 
 
+def test_profile_times_the_first_step_of_every_call():
+    """With profiling on, a call's first step runs eagerly with its timing events
+    although the captured step is current; the same bits."""
+    from moldy_amd import engine as E
+    s, e = _engine(1, False)
+    want = _run(s, e, 4, True)
+    e.profile(True)
+    for calls in (1, 2):
+        got = _run(s, e, 4, True)
+        assert all(np.array_equal(x, y) for x, y in zip(got, want))
+        assert e.profile_get("realspace")[1] == calls
+    b = E.Batch([e])
+    for schedule in (E.SCHED_GRAPH, E.SCHED_GROUPED):
+        for _ in range(2):
+            e.profile(True)
+            e.upload_state()
+            e.upload_momenta(*s.thermal_momenta(300.0, seed=4))
+            tr = b.steps(4, init_H_0=True, schedule=schedule)
+            assert np.array_equal(tr[0], want[0])
+            assert e.profile_get("realspace")[1] == 1
+    b.close()
+    e.profile(False)
+    assert np.array_equal(_run(s, e, 4, True)[0], want[0])
+    e.close()
+
+
 def test_upload_without_a_buffer_is_an_error():
     """Missing arrays are refused with a status (the copy into pinned memory
     would read them), and the engine goes on as it was."""
