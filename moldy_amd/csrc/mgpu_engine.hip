@@ -1090,7 +1090,10 @@ int mgpu_upload_state(mgpu_engine *e, const double h[9], const double *cm, const
       if (!e->have_system) return fail(e, MGPU_E_STATE, "mgpu_set_system not called");
       if (!h || !cm || (e->nmols_r && !quat)) return fail(e, MGPU_E_ARG, "bad buffers");
       HIPCHK(hipSetDevice(e->device));
+      const int version = e->geom_version;
       set_geometry(e, h);
+      // a new geometry's tables come from host arrays that end with set_geometry
+      if (e->geom_version != version) HIPCHK(hipStreamSynchronize(e->stream));
       const double *src[2] = {cm, quat};
       double *dst[2] = {e->d_cm.p, e->d_quat.p};
       const size_t n[2] = {3 * (size_t)e->nmols, 4 * (size_t)e->nmols_r};
