@@ -990,9 +990,12 @@ void mgpu::run_realspace(mgpu_engine *e) {
    a.tooclose = e->d_iflags.p + 1;
    const unsigned g = nblk, b = 256;
    bool coul = e->alpha > 0.0;
-   // FP64 sums of the FP32 pairs where the walk, which has them, was the choice
-   // by speed before the balanced kernel was: they cost nothing there
-   const bool s64 = (long)e->nsites < 16L * e->ncu;
+   // FP64 sums of the FP32 pairs below 16 sites a CU, where the walk, which has
+   // them, was the choice by speed before the balanced kernel was, and on to 32,
+   // where they cost nothing either (8,192 sites 22 us both ways; 24,000 water sites 45
+   // and 47, 48,000 81 and 85): replicas of up to 2,048 waters then share one launch
+   // (24 of them, 238 and 258 us a step: there they are enough to be issue bound)
+   const bool s64 = (long)e->nsites <= 32L * e->ncu;
    {
       ProfScope ps(e, "realspace");
       if (e->precision == MGPU_FP64) {
