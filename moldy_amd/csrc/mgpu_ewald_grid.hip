@@ -706,6 +706,14 @@ __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, co
          const int y = A.y - GB * By + j * LY + wd;
          gp[j] = sg + (lx * RX + y) * RZ + ((lz + W * ((y >> YS) & 1)) & (RZ - 1));
       }
+      // FP32: the grid less its value at the window's middle, whose force is zero:
+      // the potential (the site's own charge's for the most part) changes by a
+      // fifth over the window, and the weights' rounding meets only that
+      R mid = 0;
+      if constexpr (sizeof(R) == 4) {
+         const int y = A.y - GB * By + W / 2, z = A.z - TZ * Tz + W / 2;
+         mid = sg[((lx + W / 2) * RX + y) * RZ + ((z + W * ((y >> YS) & 1)) & (RZ - 1))];
+      }
       R a0[NJ], a1[NJ];
 #pragma unroll
       for (int j = 0; j < NJ; j++) a0[j] = a1[j] = 0;
@@ -714,7 +722,8 @@ __device__ __forceinline__ void b_g_gather(int bx, int nbx, const GGaArgs &a, co
          const T2 wx = sv[wave][i];
 #pragma unroll
          for (int j = 0; j < NJ; j++) {
-            const R gv = gp[j][i * RX * RZ];
+            R gv = gp[j][i * RX * RZ];
+            if constexpr (sizeof(R) == 4) gv -= mid;
             a0[j] += wx.x * gv;
             a1[j] += wx.y * gv;
          }
