@@ -135,7 +135,7 @@ BALANCED_CASES = tuple(c for c in CASES if c != "clay")
 @pytest.mark.parametrize("case", list(CASES))
 def test_force_calc_fp64_both_kernels(eng_mod, case, mode):
     """The per-offset walk (1), the load-balanced kernel, candidates placed
-    by piece-start bits (2) or by binary search (3), and the column-tiled
+    in windows of 2048 (2) or of 64 (3), and the column-tiled
     kernel (4), each against the oracle: same pair set, forces, energy,
     virial and close-pair count."""
     s = CASES[case]()
